@@ -167,17 +167,33 @@ __global__ __launch_bounds__(256) void bwd_gather_rows_kernel(const Src* __restr
   *reinterpret_cast<uint4*>(hc + (int64_t)q * K + (int64_t)c * CE) = v;
 }
 
-// gh from the fp32 accumulator over positions: row n = dh_acc row inv[n], or
-// zero for an inactive token.  4 values per thread.
-__global__ __launch_bounds__(256) void bwd_expand_kernel(const float* __restrict__ dh_acc, const int* __restrict__ inv,
-                                                         int N, int K, void* __restrict__ gh, int gh_dtype) {
+// gh from the fp32 accumulators over positions: row n = the sum over the vocabulary runs (in run
+// order; accumulator of run s at dh_acc + s N K) of row inv[n], or zero for an inactive token.
+// 4 values per thread; the runs' loads go out in batches of 8 ahead of the in-order adds.
+__global__ __launch_bounds__(256) void bwd_expand_kernel(const float* __restrict__ dh_acc, int n_run,
+                                                         const int* __restrict__ inv, int N, int K,
+                                                         void* __restrict__ gh, int gh_dtype) {
   const int cpr = K / 4;
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)N * cpr) return;
   const int n = (int)(e / cpr), c = (int)(e % cpr);
   const int q = inv[n];
   float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (q >= 0) v = *reinterpret_cast<const float4*>(dh_acc + (int64_t)q * K + (int64_t)c * 4);
+  if (q >= 0) {
+    const float* p = dh_acc + (int64_t)q * K + (int64_t)c * 4;
+    v = *reinterpret_cast<const float4*>(p);
+    for (int s0 = 1; s0 < n_run; s0 += 8) {
+      float4 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < n_run) x[u] = *reinterpret_cast<const float4*>(p + (int64_t)(s0 + u) * N * K);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < n_run) {
+          v.x += x[u].x; v.y += x[u].y; v.z += x[u].z; v.w += x[u].w;
+        }
+    }
+  }
   const int64_t o = (int64_t)n * K + (int64_t)c * 4;
   if (gh_dtype == kBF16) {
     bf16_t* g = static_cast<bf16_t*>(gh) + o;
@@ -1057,8 +1073,11 @@ struct GemmParams {
   int n_dw, n_dh;  // tile counts (0 when that gradient is not needed)
   void* gW;
   int gW_dtype;
-  float* dh_acc;   // dh over positions, fp32
+  float* dh_acc;   // dh over positions, fp32, one accumulator [N][K] per vocabulary run
   int dh_first;
+  int dh_split;    // vocabulary runs of a dh tile (dh_split_of); n_dh counts every run's tiles
+  int n_dh_tiles;  // dh tiles of one run
+  int dh_rows;     // rows per run, whole 32-row blocks
   float scale;     // logit scale: the stage holds dS, the products are scale * stage^T h and scale * stage W
   const int* n_act;  // active positions (device): the reduction length of dW, the rows of dh
   // dE^T = gO^T P over positions (wide scores kernel): n_de tiles, n_de_n of them along the chunk,
@@ -1332,8 +1351,9 @@ struct GemmTile {
 // positions, tok(q) their tokens):
 //   DW:  dW[v0+v][k]    = s sum_q stage[v][q] h[tok(q)][k]    (A: KTile layout, B: RTile layout)
 //   !DW: dh[tok(q)][k] += s sum_v stage[v][q] W[v0+v][k]      (A: RTile layout, B: RTile layout)
+// A dh tile covers run `run` of the chunk's vocabulary rows and adds to that run's accumulator.
 template <class T, bool DW>
-__device__ __forceinline__ void gemm_tile(const GemmParams& p, int t, char* smem) {
+__device__ __forceinline__ void gemm_tile(const GemmParams& p, int t, char* smem, int run = 0) {
   typedef GemmTile<T> G;
   constexpr int kBK = SliceK<T>::value;
   constexpr int GM = G::GM, GN = G::GN, NT = G::NT;
@@ -1356,11 +1376,15 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int t, char* smem
     gemm_loop<T, kBK, FM, FN>(acc, ta, tb, smem, (min(p.N, p.n_act[0]) + 31) & ~31, wm * (GM / G::WM),
                               wn * (GN / G::WN));
   } else {
+    const int k0 = min(p.cv, run * p.dh_rows), kn = min(p.cv - k0, p.dh_rows);
+    if (kn == 0 && !p.dh_first) return;  // an empty run of a short last chunk
     StageBRLoader<T, GM, kBK, NT> ta;
     ta.setup(p.stage, mt * GM, p.n_tb32);
+    ta.base += (int64_t)(k0 >> 5) * p.n_tb32 * 1024 * (int)sizeof(T);
     RTile<T, GN, kBK, NT> tb;
-    tb.setup(static_cast<const T*>(p.W) + (int64_t)(p.v0 - p.w_row0) * p.ldw + nt * GN, p.ldw, p.K - nt * GN, p.cv);
-    gemm_loop<T, kBK, FM, FN>(acc, ta, tb, smem, p.cv, wm * (GM / G::WM), wn * (GN / G::WN));
+    tb.setup(static_cast<const T*>(p.W) + (int64_t)(p.v0 - p.w_row0 + k0) * p.ldw + nt * GN, p.ldw, p.K - nt * GN,
+             kn);
+    gemm_loop<T, kBK, FM, FN>(acc, ta, tb, smem, kn, wm * (GM / G::WM), wn * (GN / G::WN));
   }
   const int rows = DW ? p.cv : p.N;
   const int row0 = mt * GM, col0 = nt * GN;
@@ -1374,8 +1398,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, int t, char* smem
       gemm_store<G>(acc, p.scale, static_cast<float*>(p.gW), nullptr, p.v0, rows, row0, col0, p.K, smem);
   } else {
     // dh over positions accumulates in fp32; bwd_expand_kernel writes gh
-    const float* prev = p.dh_first ? nullptr : p.dh_acc;
-    gemm_store<G, FM, FN, true>(acc, p.scale, p.dh_acc, prev, 0, rows, row0, col0, p.K, smem);
+    float* const out = p.dh_acc + (int64_t)run * p.N * p.K;
+    const float* prev = p.dh_first ? nullptr : out;
+    gemm_store<G, FM, FN, true>(acc, p.scale, out, prev, 0, rows, row0, col0, p.K, smem);
   }
 }
 
@@ -1484,12 +1509,18 @@ __global__ __launch_bounds__(GemmTile<T>::NT) void bwd_gemm_kernel(GemmParams p)
   b -= p.n_de;
   {
     // dh tiles of the active positions' row blocks only (the grid covers all
-    // of N); the active tiles are spread over every XCD
-    const int n_dh = min(p.n_dh, (p.n_act[0] + G::GM - 1) / G::GM * p.n_n);
-    if (b < n_dh) {
+    // of N); the active tiles are spread over every XCD.  With the vocabulary
+    // split in runs, a run's tiles are consecutive, so an XCD works on few runs.
+    const int n_t = min(p.n_dh_tiles, (p.n_act[0] + G::GM - 1) / G::GM * p.n_n);
+    if (b < n_t * p.dh_split) {
+      int t = xcd_swizzle(b, n_t * p.dh_split), run = 0;
+      if (p.dh_split > 1) {
+        run = t / n_t;
+        t -= run * n_t;
+      }
       int r, c;
-      grouped_tile(b, n_dh / p.n_n, p.n_n, &r, &c);
-      gemm_tile<T, false>(p, r * p.n_n + c, smem);
+      grouped_order(t, n_t / p.n_n, p.n_n, &r, &c);
+      gemm_tile<T, false>(p, r * p.n_n + c, smem, run);
     }
   }
 }
@@ -1621,6 +1652,7 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
   T* hqc = reinterpret_cast<T*>(ws + plan.off_hqc);
   float* multp = f8 ? reinterpret_cast<float*>(ws + plan.off_mult) : nullptr;
   const bool need_stage = p.gh || p.gW;
+  const int dh_split = p.gW ? plan.dh_split_w : plan.dh_split_h;
   const bool gemm_de = pstage && p.gE;  // dE^T = gO^T P as tiles of the gradient GEMM launch
   // every chunk has a gradient GEMM launch: the W packing of the scores kernel rides on them
   const bool fold_pack = !f8 && (need_stage || gemm_de);
@@ -1751,7 +1783,10 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
       gp.cv = cv;
       gp.n_n = (p.K + plan.GN - 1) / plan.GN;
       gp.n_dw = p.gW ? ((cv + plan.GM - 1) / plan.GM) * gp.n_n : 0;
-      gp.n_dh = p.gh ? ((p.N + plan.GM - 1) / plan.GM) * gp.n_n : 0;
+      gp.dh_split = dh_split;
+      gp.dh_rows = ((cv + dh_split - 1) / dh_split + 31) & ~31;
+      gp.n_dh_tiles = p.gh ? ((p.N + plan.GM - 1) / plan.GM) * gp.n_n : 0;
+      gp.n_dh = gp.n_dh_tiles * dh_split;
       gp.n_de_n = (cv + plan.GN - 1) / plan.GN;
       gp.de_split = de_split(plan.N_pad);
       gp.n_de = gemm_de ? ((plan.DP + plan.GM - 1) / plan.GM) * gp.n_de_n * gp.de_split : 0;
@@ -1815,7 +1850,8 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
     const int64_t ng = (int64_t)p.N * (p.K / 4);
     if (ng > 0) {
       timing_begin(kKindBwdExpand, stream);
-      bwd_expand_kernel<<<(int)((ng + 255) / 256), 256, 0, stream>>>(dh_acc, inv, p.N, p.K, p.gh, p.gh_dtype);
+      bwd_expand_kernel<<<(int)((ng + 255) / 256), 256, 0, stream>>>(dh_acc, dh_split, inv, p.N, p.K, p.gh,
+                                                                            p.gh_dtype);
       timing_end(kKindBwdExpand, stream);
       if ((e = hipGetLastError()) != hipSuccess) return e;
     }
@@ -1925,7 +1961,18 @@ bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chu
   plan->off_pb = off;
   off += align256((size_t)plan->n_gpart * c * 4);
   plan->off_dh = off;
-  if (plan->dh_acc) off += align256((size_t)N * K * 4);
+  plan->dh_split_w = plan->dh_split_h = 1;
+  if (plan->dh_acc) {
+    // a two-byte GEMM tile holds a CU, an fp32 one half; a tile's overheads in reduction slices
+    // (0.6 us, fp32 1 us)
+    const int64_t n_n = (K + GN - 1) / GN, sl = two ? SliceK<bf16_t>::value : SliceK<float>::value;
+    const int64_t n_dw = (c + GM - 1) / GM * n_n, n_dh = (N + GM - 1) / GM * n_n, acc = N * K * 4;
+    const int slots = two ? 256 : 512, o_dw = two ? 8 : 5, o_dh = two ? 12 : 7;
+    plan->dh_split_w = dh_split_of(n_dw, (N + sl - 1) / sl, n_dh, c / sl, slots, o_dw, o_dh, acc);
+    plan->dh_split_h = dh_split_of(0, 0, n_dh, c / sl, slots, o_dw, o_dh, acc);
+    const int s = plan->dh_split_w > plan->dh_split_h ? plan->dh_split_w : plan->dh_split_h;
+    off += align256((size_t)acc * s);
+  }
   plan->off_gO = off;
   off += align256((size_t)plan->N_pad * DP * tb);
   plan->off_gOt = off;

@@ -888,12 +888,15 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
 // go to the XCDs round-robin, xcd_swizzle gives each XCD a contiguous range of
 // the tile order, and the order walks G-row column strips.
 template <int G = 4>
-__device__ __forceinline__ void grouped_tile(int b, int R, int Q, int* row, int* col) {
-  const int t = xcd_swizzle(b, R * Q);
+__device__ __forceinline__ void grouped_order(int t, int R, int Q, int* row, int* col) {
   const int group = t / (G * Q), first = group * G;
   const int gsize = min(R - first, G);
   *row = first + (t % (G * Q)) % gsize;
   *col = (t % (G * Q)) / gsize;
+}
+template <int G = 4>
+__device__ __forceinline__ void grouped_tile(int b, int R, int Q, int* row, int* col) {
+  grouped_order<G>(xcd_swizzle(b, R * Q), R, Q, row, col);
 }
 
 // An LDS ring of NS slots whose stages are not issued at a uniform rate: the

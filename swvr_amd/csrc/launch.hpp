@@ -150,6 +150,8 @@ struct BwdPlan {
   int hS8;               // e4m3 scores: reduction slices of the packed e4m3 h and W (K8 / 2 pairs)
   size_t off_hqc, off_mult;
   size_t off_pstage;     // P stage (wide scores kernel), the dS stage's layout
+  // vocabulary runs each dh tile's reduction is split over (dh_split_of), beside dW tiles and alone
+  int dh_split_w, dh_split_h;
 };
 
 // Scores kernels of the backward (BwdPlan::kind).
@@ -161,6 +163,51 @@ constexpr int kDeSplit = 8;
 inline int de_split(int64_t n_pad) {
   const int64_t s = n_pad / 2048;
   return s < 1 ? 1 : s > kDeSplit ? kDeSplit : (int)s;
+}
+
+// Runs of a chunk's vocabulary rows that each dh tile is split over, every run a piece of the
+// gradient GEMM launch with an fp32 accumulator of its own (summed in run order when gh is
+// written).  A launch has n_dw dW tiles of s_dw reduction slices and n_dh dh tiles of s_dh; with
+// few tokens the dh tiles are few and long (8 tiles of 256 slices beside 128 of 16 at 512 tokens,
+// K = 1024), and the launch waits for them with most CUs idle.  The split minimises the launch's
+// duration when `slots` workgroups run at a time, dW tiles dealt first, with o_dw / o_dh slices'
+// worth of time per tile for its prologue and stores: a run that ends in a read-modify-write of
+// its accumulator costs more than a dW tile.  Runs keep at least 8 slices, the accumulators beyond
+// the first (acc_bytes each) stay within kDhSplitBytes, and a split must gain 5%.
+// Measured, the whole call, whole tiles against split: N = 2048, K = 1024, V = 151936, gh alone (32 dh
+// tiles per chunk, 8 runs) 4.65 -> 2.63 ms; N = 500, K = 1024, V = 32000, every gradient (8 dh and 128
+// dW tiles, 16 runs) 1.02 -> 0.53 ms; N = 2048, K = 2048, V = 65536 (64 and 256, 4 runs) 3.48 -> 2.95.
+constexpr int64_t kDhSplitBytes = (int64_t)64 << 20;
+inline int dh_split_of(int64_t n_dw, int64_t s_dw, int64_t n_dh, int64_t s_dh, int slots, int o_dw, int o_dh,
+                       int64_t acc_bytes) {
+  if (n_dh <= 0) return 1;
+  const int64_t a = s_dw + o_dw, q = n_dw / slots, r = n_dw % slots;
+  auto span = [&](int64_t s) {
+    const int64_t jobs = n_dh * s, b = (s_dh + s - 1) / s + o_dh;
+    // r slots are free at (q + 1) a, the others at q a: the earliest end of all jobs of length b
+    auto fits = [&](int64_t t) {
+      const int64_t x = t >= (q + 1) * a ? (t - (q + 1) * a) / b : 0, y = t >= q * a ? (t - q * a) / b : 0;
+      return r * x + (slots - r) * y >= jobs;
+    };
+    const int64_t lo = (q + 1) * a, rounds = jobs / slots + 2;
+    int64_t best = INT64_MAX;
+    for (int64_t i = 0; i <= rounds; ++i) {
+      const int64_t t0 = q * a + i * b, t1 = (q + 1) * a + i * b;
+      if (fits(t0) && t0 < best) best = t0;
+      if (fits(t1) && t1 < best) best = t1;
+    }
+    return r > 0 && best < lo ? lo : best;
+  };
+  int64_t best = span(1) * 95 / 100;
+  int split = 1;
+  for (int s = 2; s <= 64 && s_dh / s >= 8 && (s - 1) * acc_bytes <= kDhSplitBytes; s *= 2) {
+    const int64_t t = span(s);
+    if (t < best) {
+      best = t;
+      split = s;
+    }
+  }
+  return split;
 }
 
 // w_f32: W is stored in fp32 and needs a row-major copy in the compute dtype
