@@ -47,49 +47,73 @@ __device__ __forceinline__ void store_as(void* base, int64_t idx, int dtype, flo
 // positions 0 .. n_act - 1; positions n_act .. N_pad - 1 are padding.
 
 // delta = rowsum(O * gO) - gLSE (swvr/chunked.py:113-114) and the active flag,
-// one thread per token.  gO enters the sum rounded to the compute dtype T, as it
+// 16 lanes per token (64-byte runs of its rows).  One thread per token read a
+// row per lane, serially: 16 us at 500 tokens, D = 64, and 82 us at 32768, D = 256;
+// 16 lanes take 3.5 and 14 us.  gO enters the sum rounded to the compute dtype T, as it
 // enters dP = gO E^T: the reference sums it unrounded, which leaves dP - delta,
 // where those nearly cancel (one vocabulary row, or one row with all of P),
 // with the rounding error of gO alone (gh and gb then miss the fp32 formula by
 // 2-7% in bf16 at V = 1, D = 300; 0.2% with the rounded sum).  Elsewhere the two
 // sums agree to that rounding.
+constexpr int kDeltaLanes = 16;
 template <class T>
 __global__ __launch_bounds__(256) void bwd_delta_kernel(const float* __restrict__ O, const float* __restrict__ gO,
                                                         const float* __restrict__ glse, int N, int D,
                                                         float* __restrict__ delta, int* __restrict__ flag) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int n = (int)(e / kDeltaLanes), c = (int)(e % kDeltaLanes);
+  const bool in = n < N;
   float s = 0.f;
   bool nz = false;
-  for (int k = 0; k < D; ++k) {
-    const float g = gO[(int64_t)n * D + k];
-    s += O[(int64_t)n * D + k] * to_float(from_float<T>(g));
-    nz |= g != 0.f;
+  if (in)
+    for (int k = c; k < D; k += kDeltaLanes) {
+      const float g = gO[(int64_t)n * D + k];
+      s += O[(int64_t)n * D + k] * to_float(from_float<T>(g));
+      nz |= g != 0.f;
+    }
+#pragma unroll
+  for (int o = kDeltaLanes / 2; o > 0; o >>= 1) {
+    s += __shfl_xor(s, o);
+    nz |= __shfl_xor((int)nz, o) != 0;
   }
+  if (!in || c != 0) return;
   s -= glse[n];
   delta[n] = s;
   flag[n] = nz || glse[n] != 0.f || s != 0.f;  // NaN != 0
 }
 
 // Order-preserving compaction of the active tokens: idx[q] = token of
-// position q, inv[n] = position of token n or -1, n_act[0] = count.  One
-// workgroup; each thread scans IT consecutive tokens per round.
-__global__ __launch_bounds__(1024) void bwd_compact_kernel(const int* __restrict__ flag, int N, int* __restrict__ idx,
-                                                           int* __restrict__ inv, int* __restrict__ n_act) {
-  constexpr int IT = 16;
+// position q, inv[n] = position of token n or -1, n_act[0] = count.  Workgroup
+// b takes `per` tokens (a multiple of 1024) from b * per on, after counting the
+// flags before them itself, so no workgroup waits for another; compact_tokens
+// keeps the grid at 256 or fewer, which bounds those reads to 512 bytes a token.
+// One workgroup scanning every token took 23 us for 16384 tokens and 51 for 32768
+// (scattered idx and inv stores, rounds in series); this takes 5 and 6.
+__global__ __launch_bounds__(1024) void bwd_compact_kernel(const int* __restrict__ flag, int N, int per,
+                                                           int* __restrict__ idx, int* __restrict__ inv,
+                                                           int* __restrict__ n_act) {
   __shared__ int wsum[16];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int64_t first = (int64_t)blockIdx.x * per;  // < N
   int carry = 0;
-  for (int base = 0; base < N; base += 1024 * IT) {
-    const int n0 = base + t * IT;
-    int f[IT];
+  {
     int cnt = 0;
-#pragma unroll
-    for (int i = 0; i < IT; ++i) {
-      f[i] = n0 + i < N ? flag[n0 + i] : 0;
-      cnt += f[i];
+    for (int64_t i = (int64_t)t * 4; i < first; i += 4096) {  // first is a multiple of 1024
+      const int4 x = *reinterpret_cast<const int4*>(flag + i);
+      cnt += (x.x + x.y) + (x.z + x.w);
     }
-    int x = cnt;  // inclusive scan over the wave
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+    if (lane == 0) wsum[w] = cnt;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) carry += wsum[j];
+    __syncthreads();
+  }
+  for (int64_t n0 = first; n0 < first + per && n0 < N; n0 += 1024) {
+    const int64_t n = n0 + t;
+    const int f = n < N ? flag[n] : 0;
+    int x = f;  // inclusive scan over the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int y = __shfl_up(x, o);
@@ -103,19 +127,13 @@ __global__ __launch_bounds__(1024) void bwd_compact_kernel(const int* __restrict
       before += j < w ? wsum[j] : 0;
       total += wsum[j];
     }
-    int q = carry + before + x - cnt;
-#pragma unroll
-    for (int i = 0; i < IT; ++i) {
-      const int n = n0 + i;
-      if (n < N) {
-        inv[n] = f[i] ? q : -1;
-        if (f[i]) idx[q++] = n;
-      }
-    }
+    const int q = carry + before + x - f;
+    if (n < N) inv[n] = f ? q : -1;
+    if (f) idx[q] = (int)n;
     carry += total;
     __syncthreads();  // wsum is rewritten next round
   }
-  if (t == 0) n_act[0] = carry;
+  if (t == 0 && first + per >= N) n_act[0] = carry;
 }
 
 // The token-side operands of the scores kernel over positions: gO rounded to
@@ -1660,19 +1678,20 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
   {
     // delta, the active tokens, and the token-side operands over positions
     timing_begin(kKindBwdDelta, stream);
-    bwd_delta_kernel<T><<<(p.N + 255) / 256, 256, 0, stream>>>(p.O, p.gO, p.glse, p.N, p.D, delta, flag);
-    bwd_compact_kernel<<<1, 1024, 0, stream>>>(flag, p.N, idx, inv, n_act);
+    bwd_delta_kernel<T><<<(unsigned)(((int64_t)p.N * kDeltaLanes + 255) / 256), 256, 0, stream>>>(p.O, p.gO, p.glse, p.N, p.D, delta, flag);
+    if ((e = compact_tokens(flag, p.N, idx, inv, n_act, stream)) != hipSuccess) return e;
     const int64_t n = (int64_t)plan.N_pad * plan.DP;
     bwd_pack_kernel<T><<<(int)((n + 255) / 256), 256, 0, stream>>>(p.gO, p.lse, delta, idx, n_act, p.D,
                                                                    (int)plan.N_pad, plan.DP, plan.BM, gOp, gOt,
                                                                    lsed);
     timing_end(kKindBwdDelta, stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int64_t nv = (int64_t)plan.V_pad * plan.DP;
+    const int64_t nv = (int64_t)plan.V_pad * (plan.DP / 8);
+    const T* E = static_cast<const T*>(p.E);
     timing_begin(kKindPack, stream);
-    pack_vocab_kernel<T><<<(int)((nv + 255) / 256), 256, 0, stream>>>(
-        static_cast<const T*>(p.E), p.lde, p.bias, p.V, p.D, plan.V_pad, plan.DP, Ep, biasp, p.h_scale, p.w_scale,
-        p.scale, multp);
+    pack_vocab_kernel<T><<<(unsigned)((nv + 255) / 256), 256, 0, stream>>>(E, p.lde, p.bias, p.V, p.D, plan.V_pad,
+                                                                           plan.DP, rows_vec16(E, p.lde), Ep, biasp,
+                                                                           p.h_scale, p.w_scale, p.scale, multp);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (p.K > 0) {
       const int64_t nh = plan.N_pad * (p.K / (16 / (int)sizeof(T)));
@@ -1877,7 +1896,9 @@ size_t dtype_bytes(int dtype) { return dtype == kF32 ? 4 : 2; }
 }  // namespace
 
 hipError_t compact_tokens(const int* flag, int N, int* idx, int* inv, int* n_act, hipStream_t stream) {
-  bwd_compact_kernel<<<1, 1024, 0, stream>>>(flag, N, idx, inv, n_act);
+  // the grid of bwd_compact_kernel: whole rounds of 1024 tokens over at most 256 workgroups (N > 0)
+  const int64_t rounds = ((int64_t)N + 1023) / 1024, per = (rounds + 255) / 256 * 1024;
+  bwd_compact_kernel<<<(unsigned)((N + per - 1) / per), 1024, 0, stream>>>(flag, N, (int)per, idx, inv, n_act);
   return hipGetLastError();
 }
 

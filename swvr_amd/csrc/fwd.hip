@@ -80,31 +80,58 @@ using FwdCfg = typename std::conditional<F8, FwdTileF8<DP>, FwdTile<T, DP>>::typ
 // With w_scale set (the e4m3 forward) the bias goes out as (bias, multiplier)
 // pairs, multiplier = logit_scale * h_scale * w_scale[v] (0 past V): the
 // factor that turns the e4m3 dot product into a score.
-template <class T>
+// One workgroup per 32 columns of a tile: E's rows are read along d (64-byte
+// runs, any alignment of E), E^T rows written as whole 16-byte chunks.  Bound by
+// its traffic (E in, E^T out); one thread per element, which read E a row per
+// lane, took 53 us at V = 151936, D = 64 and this 15 us.
+template <class T, int BV>
 __global__ __launch_bounds__(256) void pack_et_kernel(const T* __restrict__ E, int64_t lde,
                                                       const float* __restrict__ bias, int V, int D, int V_pad,
-                                                      int DP, int BV, T* __restrict__ Et, float* __restrict__ biasp,
+                                                      int DP, T* __restrict__ Et, float* __restrict__ biasp,
                                                       const float* __restrict__ h_scale,
                                                       const float* __restrict__ w_scale, float logit_scale) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < (int64_t)V_pad * DP) {
-    const int64_t tile = e / ((int64_t)DP * BV);
-    const int rem = (int)(e - tile * DP * BV);
-    const int d = rem / BV, p = rem % BV;
-    const int64_t v = tile * BV + pe_row(p);
-    Et[e] = (v < V && d < D) ? E[v * lde + d] : (T)0.f;
-  }
-  if (e < V_pad) {
-    const float b = e < V ? (bias ? bias[e] : 0.f) : kNegInf;
-    if (w_scale) {
-      biasp[2 * e] = b;
-      biasp[2 * e + 1] = e < V ? logit_scale * h_scale[0] * w_scale[e] : 0.f;
-    } else {
-      biasp[e] = b;
+  constexpr int CE = 16 / (int)sizeof(T);
+  constexpr int LS = 32 + 4 / (int)sizeof(T);  // elements per LDS row (one 4-byte word of padding)
+  __shared__ T tile[BV * LS];
+  const int ndb = DP / 32;
+  const int vt = blockIdx.x / ndb, d0 = (blockIdx.x % ndb) * 32, v0 = vt * BV;
+  const int t = threadIdx.x;
+  {
+    const int d = d0 + t % 32;
+    T x[BV / 8];  // every load issued before the first is used
+#pragma unroll
+    for (int i = 0; i < BV / 8; ++i) {
+      const int v = v0 + i * 8 + t / 32;
+      x[i] = v < V && d < D ? E[(int64_t)v * lde + d] : (T)0.f;
     }
+#pragma unroll
+    for (int i = 0; i < BV / 8; ++i) tile[(i * 8 + t / 32) * LS + t % 32] = x[i];
   }
+  __syncthreads();
+  T* out = Et + ((int64_t)vt * DP + d0) * BV;
+#pragma unroll
+  for (int i = 0; i < BV * 32 / CE / 256; ++i) {
+    const int c = i * 256 + t;  // 16-byte chunk of the 32 rows
+    const int d = c / (BV / CE), p = (c % (BV / CE)) * CE;
+    T q[CE];
+#pragma unroll
+    for (int j = 0; j < CE; ++j) q[j] = tile[pe_row(p + j) * LS + d];
+    uint4 u;
+    __builtin_memcpy(&u, q, 16);
+    *reinterpret_cast<uint4*>(out + (int64_t)c * CE) = u;
+  }
+  if (d0 == 0)
+    for (int i = t; i < BV; i += 256) {
+      const int e = v0 + i;
+      const float b = e < V ? (bias ? bias[e] : 0.f) : kNegInf;
+      if (w_scale) {
+        biasp[2 * (int64_t)e] = b;
+        biasp[2 * (int64_t)e + 1] = e < V ? logit_scale * h_scale[0] * w_scale[e] : 0.f;
+      } else {
+        biasp[e] = b;
+      }
+    }
 }
-
 
 template <class T, int DP, bool F8 = false>
 __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdParams p) {
@@ -569,69 +596,114 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
 // one kernel merges the forward's own partials ([n_part][DP][N], token
 // fastest) and vocabulary shards' ([S][N][D]).  With m_out set, it writes the
 // merged partial (M, L and the unnormalised acc, [N][D]) instead of O / LSE.
-// One thread per (d, n) with n fastest; the d = 0 thread of a row also writes
-// its LSE (or M, L).
-// Merge of one (row, column) over n_part partials: m / l of partial q at
-// pm[q * sml] / pl[q * sml], its acc at pa[q * sp] (read when has_d).  The
-// loads go out in batches of 8 ahead of the arithmetic, which runs in partial
-// order, so the merge waits for memory once per batch, not once per partial.
+// A thread merges DT consecutive columns of a row (n fastest over the threads), so the row's m and l
+// are read and exponentiated once per DT columns; the d = 0 threads also write their row's LSE (or M, L).
+//
+// Merge over n_part partials by a workgroup of G thread rows x 256 / G columns (G = 32: x 32): m / l
+// of partial q at pm[q * sml] / pl[q * sml], its acc of column i at pa[q * sp + i * sd] (i < nd).  Each
+// thread row merges a contiguous run of the partials, loads going out in batches of 8 ahead of the
+// arithmetic, and the runs' sums are added in run order, so the result has a fixed order.
+//   G = 32, DT = 1: few elements and many partials, where the merge is bound by the latency of a
+//   run's loads: one token's 594 partials take 11 us (102 us in one run per element).
+//   G = 4, DT = 4: many partials, many elements: 2048 tokens, D = 128, 128 partials 74 us (G = 1: 96).
+//   G = 1, DT = 4: few partials: bound by their bytes.  16384 tokens, D = 64, 32 partials 50 us
+//   (G = 4: 55; one column per thread, with four loads of m and l for each of acc: 79).
+template <int G>
+struct MergeWidth {
+  static constexpr int value = G == 32 ? 32 : 256 / G;
+};
+
+template <int G, int DT>
 __device__ __forceinline__ void merge_partials(const float* __restrict__ pm, const float* __restrict__ pl,
                                                const float* __restrict__ pa, int n_part, int64_t sml, int64_t sp,
-                                               bool has_d, float* M_, float* L_, float* a_) {
-  constexpr int B = 8;
+                                               int64_t sd, bool live, int nd, float* M_, float* L_, float (&a_)[DT]) {
+  constexpr int B = 8, CW = MergeWidth<G>::value;
+  __shared__ float sm[G][CW], sl[G][CW], sa[DT][G][CW];
+  const int g = threadIdx.x / CW, c = threadIdx.x % CW;
+  const int run = (n_part + G - 1) / G;
+  const int q_begin = min(n_part, g * run), q_end = live ? min(n_part, q_begin + run) : q_begin;
   float M = kNegInf;
-  for (int q0 = 0; q0 < n_part; q0 += B) {
+  for (int q0 = q_begin; q0 < q_end; q0 += B) {
     float x[B];
 #pragma unroll
-    for (int u = 0; u < B; ++u) x[u] = q0 + u < n_part ? pm[(q0 + u) * sml] : kNegInf;
+    for (int u = 0; u < B; ++u) x[u] = q0 + u < q_end ? pm[(q0 + u) * sml] : kNegInf;
 #pragma unroll
     for (int u = 0; u < B; ++u) M = fmaxf(M, x[u]);
   }
+  if constexpr (G > 1) {
+    sm[g][c] = M;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < G; ++i) M = fmaxf(M, sm[i][c]);
+  }
   const float shift = M == kNegInf ? 0.f : M;
-  float L = 0.f, a = 0.f;
-  for (int q0 = 0; q0 < n_part; q0 += B) {
-    float xm[B], xl[B], xa[B];
+  float L = 0.f;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) a_[i] = 0.f;
+  for (int q0 = q_begin; q0 < q_end; q0 += B) {
+    float xm[B], xl[B], xa[B][DT];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-      const bool in = q0 + u < n_part;
+      const bool in = q0 + u < q_end;
       xm[u] = in ? pm[(q0 + u) * sml] : 0.f;
       xl[u] = in ? pl[(q0 + u) * sml] : 0.f;
-      xa[u] = in && has_d ? pa[(q0 + u) * sp] : 0.f;
+#pragma unroll
+      for (int i = 0; i < DT; ++i) xa[u][i] = in && i < nd ? pa[(q0 + u) * sp + i * sd] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < B; ++u)
-      if (q0 + u < n_part) {
+      if (q0 + u < q_end) {
         const float wq = expf(xm[u] - shift);
         L += xl[u] * wq;
-        if (has_d) a += xa[u] * wq;
+#pragma unroll
+        for (int i = 0; i < DT; ++i) a_[i] += xa[u][i] * wq;
       }
+  }
+  if constexpr (G > 1) {
+    sl[g][c] = L;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) sa[i][g][c] = a_[i];
+    __syncthreads();
+    L = 0.f;
+#pragma unroll
+    for (int j = 0; j < G; ++j) L += sl[j][c];
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      a_[i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < G; ++j) a_[i] += sa[i][j][c];
+    }
   }
   *M_ = M;
   *L_ = L;
-  *a_ = a;
 }
 
-__global__ __launch_bounds__(256) void fwd_combine_kernel(const float* __restrict__ part_m,
-                                                          const float* __restrict__ part_l,
-                                                          const float* __restrict__ part_acc, int n_part, int N,
-                                                          int D, int64_t sp, int64_t sd, int64_t sn,
-                                                          float* __restrict__ O, int64_t ldo, float* __restrict__ lse,
-                                                          float* __restrict__ m_out, float* __restrict__ l_out) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int Dw = D > 0 ? D : 1;
-  if (e >= (int64_t)N * Dw) return;
-  const int d = (int)(e / N), n = (int)(e % N);
-  float M, L, a;
-  merge_partials(part_m + n, part_l + n, part_acc + d * sd + n * sn, n_part, N, sp, d < D, &M, &L, &a);
-  if (m_out) {
-    if (d < D) O[(int64_t)n * ldo + d] = a;
-    if (d == 0) {
+// Thread rows G of a merge (DT = 1 with 32, else 4).
+int combine_rows(int64_t elements, int n_part) { return n_part < 64 ? 1 : elements <= 65536 ? 32 : 4; }
+
+template <int G, int DT>
+__global__ __launch_bounds__(G * MergeWidth<G>::value) void fwd_combine_kernel(
+    const float* __restrict__ part_m, const float* __restrict__ part_l, const float* __restrict__ part_acc, int n_part,
+    int N, int D, int64_t sp, int64_t sd, int64_t sn, float* __restrict__ O, int64_t ldo, float* __restrict__ lse,
+    float* __restrict__ m_out, float* __restrict__ l_out) {
+  constexpr int CW = MergeWidth<G>::value;
+  const int64_t e = (int64_t)blockIdx.x * CW + threadIdx.x % CW;
+  const int nb = D > 0 ? (D + DT - 1) / DT : 1;
+  const bool live = e < (int64_t)N * nb;
+  const int d = live ? (int)(e / N) * DT : 0, n = live ? (int)(e % N) : 0;
+  float M, L, a[DT];
+  merge_partials<G, DT>(part_m + n, part_l + n, part_acc + d * sd + n * sn, n_part, N, sp, sd, live, D - d, &M, &L, a);
+  if (!live || threadIdx.x >= CW) return;
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+    if (d + i < D) O[(int64_t)n * ldo + d + i] = m_out ? a[i] : a[i] / L;
+  if (d == 0) {
+    if (m_out) {
       m_out[n] = M;
       l_out[n] = L;
+    } else {
+      lse[n] = M + logf(L);
     }
-  } else {
-    if (d < D) O[(int64_t)n * ldo + d] = a / L;
-    if (d == 0) lse[n] = M + logf(L);
   }
 }
 
@@ -639,27 +711,59 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const float* __restric
 // of its position inv[n] (WV x n_split partials of n_tb x BM rows each, n_tb and
 // n_split at n_act[3], n_act[4]); a token outside the active set gets an O row
 // of 0 and LSE 0.
-__global__ __launch_bounds__(256) void fwd_combine_active_kernel(
+template <int G, int DT>
+__global__ __launch_bounds__(G * MergeWidth<G>::value) void fwd_combine_active_kernel(
     const float* __restrict__ part_m, const float* __restrict__ part_l, const float* __restrict__ part_acc,
     const int* __restrict__ inv, const int* __restrict__ n_act, int BM, int WV, int N, int D, int DP,
     float* __restrict__ O, int64_t ldo, float* __restrict__ lse) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int Dw = D > 0 ? D : 1;
-  if (e >= (int64_t)N * Dw) return;
-  const int d = (int)(e / N), n = (int)(e % N);
-  const int q = inv[n];
-  if (q < 0) {
-    if (d < D) O[(int64_t)n * ldo + d] = 0.f;
-    if (d == 0) lse[n] = 0.f;
-    return;
-  }
+  constexpr int CW = MergeWidth<G>::value;
+  const int64_t e = (int64_t)blockIdx.x * CW + threadIdx.x % CW;
+  const int nb = D > 0 ? (D + DT - 1) / DT : 1;
+  const bool in = e < (int64_t)N * nb;
+  const int d = in ? (int)(e / N) * DT : 0, n = in ? (int)(e % N) : 0;
+  const int q = in ? inv[n] : -1, qc = q < 0 ? 0 : q;
   const int tb = n_act[3], sp = n_act[4];
   const int64_t rows = (int64_t)tb * BM;
-  float M, L, a;
-  merge_partials(part_m + q, part_l + q, part_acc + d * rows + q, WV * sp, rows, (int64_t)DP * rows, d < D, &M, &L,
-                 &a);
-  if (d < D) O[(int64_t)n * ldo + d] = a / L;
-  if (d == 0) lse[n] = M + logf(L);
+  float M, L, a[DT];
+  merge_partials<G, DT>(part_m + qc, part_l + qc, part_acc + d * rows + qc, WV * sp, rows, (int64_t)DP * rows, rows,
+                        q >= 0, D - d, &M, &L, a);
+  if (!in || threadIdx.x >= CW) return;
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+    if (d + i < D) O[(int64_t)n * ldo + d + i] = q >= 0 ? a[i] / L : 0.f;
+  if (d == 0) lse[n] = q >= 0 ? M + logf(L) : 0.f;
+}
+
+// Workgroups of a merge of N rows x D columns.
+template <int G, int DT>
+unsigned combine_blocks(int N, int D) {
+  constexpr int CW = MergeWidth<G>::value;
+  return (unsigned)(((int64_t)N * (D > 0 ? (D + DT - 1) / DT : 1) + CW - 1) / CW);
+}
+
+template <class F>
+void dispatch_combine(int64_t elements, int n_part, F&& go) {
+  switch (combine_rows(elements, n_part)) {
+    case 1: go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>()); break;
+    case 4: go(std::integral_constant<int, 4>(), std::integral_constant<int, 4>()); break;
+    default: go(std::integral_constant<int, 32>(), std::integral_constant<int, 1>()); break;
+  }
+}
+
+// Merge launch over n_part partials of N rows x D columns (see fwd_combine_kernel).
+hipError_t launch_combine(const float* m, const float* l, const float* acc, int n_part, int N, int D, int64_t sp,
+                          int64_t sd, int64_t sn, float* O, int64_t ldo, float* lse, float* m_out, float* l_out,
+                          hipStream_t stream) {
+  if (N == 0) return hipSuccess;
+  timing_begin(kKindFwdCombine, stream);
+  auto go = [&](auto g, auto dt) {
+    constexpr int G = decltype(g)::value, DT = decltype(dt)::value;
+    fwd_combine_kernel<G, DT><<<combine_blocks<G, DT>(N, D), G * MergeWidth<G>::value, 0, stream>>>(
+        m, l, acc, n_part, N, D, sp, sd, sn, O, ldo, lse, m_out, l_out);
+  };
+  dispatch_combine((int64_t)N * D, n_part, go);
+  timing_end(kKindFwdCombine, stream);
+  return hipGetLastError();
 }
 
 // The active-token forward's token blocks and vocabulary splits (active_grid)
@@ -791,10 +895,13 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // E^T tiles and the bias of one D-slice (p.E, p.D: the slice's columns).
 template <class T>
 hipError_t pack_et(const FwdParams& p, const FwdPlan& plan, hipStream_t stream) {
-  const int64_t n = (int64_t)plan.V_pad * plan.DP;
+  constexpr int BV = FwdTile<T, 32>::BV;  // one per dtype
+  if (plan.BV != BV) return hipErrorInvalidValue;
+  const int64_t blocks = (int64_t)plan.n_vt * (plan.DP / 32);
+  if (blocks == 0) return hipSuccess;
   timing_begin(kKindPack, stream);
-  pack_et_kernel<T><<<(int)((n + 255) / 256), 256, 0, stream>>>(
-      static_cast<const T*>(p.E), p.lde, p.bias, p.V, p.D, plan.V_pad, plan.DP, plan.BV,
+  pack_et_kernel<T, BV><<<(unsigned)blocks, 256, 0, stream>>>(
+      static_cast<const T*>(p.E), p.lde, p.bias, p.V, p.D, plan.V_pad, plan.DP,
       const_cast<T*>(static_cast<const T*>(p.Ep)), const_cast<float*>(p.biasp), p.h_scale, p.w_scale, p.scale);
   timing_end(kKindPack, stream);
   return hipGetLastError();
@@ -941,13 +1048,9 @@ hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, flo
     }
     if (e != hipSuccess) return e;
     // every pass computes the same scores, so each writes the same lse (m, l); O gets its columns
-    timing_begin(kKindFwdCombine, stream);
-    const int64_t n_threads = (int64_t)p.N * (q.D > 0 ? q.D : 1);
-    fwd_combine_kernel<<<(int)((n_threads + 255) / 256), 256, 0, stream>>>(
-        p.part_m, p.part_l, p.part_acc, plan.n_part, p.N, q.D, (int64_t)plan.DP * p.N, p.N, 1, O ? O + d0 : nullptr,
-        D, lse, m_out, l_out);
-    timing_end(kKindFwdCombine, stream);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    e = launch_combine(p.part_m, p.part_l, p.part_acc, plan.n_part, p.N, q.D, (int64_t)plan.DP * p.N, p.N, 1,
+                       O ? O + d0 : nullptr, D, lse, m_out, l_out, stream);
+    if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }
@@ -1045,9 +1148,12 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
     }
     if (e != hipSuccess) return e;
     timing_begin(kKindFwdCombine, stream);
-    const int64_t n_threads = (int64_t)p.N * (q.D > 0 ? q.D : 1);
-    fwd_combine_active_kernel<<<(int)((n_threads + 255) / 256), 256, 0, stream>>>(
-        p.part_m, p.part_l, p.part_acc, inv, n_act, plan.BM, plan.WV, p.N, q.D, plan.DP, O + d0, D, lse);
+    auto go = [&](auto g, auto dt) {
+      constexpr int G = decltype(g)::value, DT = decltype(dt)::value;
+      fwd_combine_active_kernel<G, DT><<<combine_blocks<G, DT>(p.N, q.D), G * MergeWidth<G>::value, 0, stream>>>(
+          p.part_m, p.part_l, p.part_acc, inv, n_act, plan.BM, plan.WV, p.N, q.D, plan.DP, O + d0, D, lse);
+    };
+    dispatch_combine((int64_t)p.N * q.D, plan.n_part, go);
     timing_end(kKindFwdCombine, stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -1056,13 +1162,7 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
 
 hipError_t shard_combine(int S, int N, int D, const float* m, const float* l, const float* acc, float* O, float* lse,
                          hipStream_t stream) {
-  const int64_t n_threads = (int64_t)N * (D > 0 ? D : 1);
-  if (n_threads == 0) return hipSuccess;
-  timing_begin(kKindFwdCombine, stream);
-  fwd_combine_kernel<<<(int)((n_threads + 255) / 256), 256, 0, stream>>>(m, l, acc, S, N, D, (int64_t)N * D, 1, D, O,
-                                                                         D, lse, nullptr, nullptr);
-  timing_end(kKindFwdCombine, stream);
-  return hipGetLastError();
+  return launch_combine(m, l, acc, S, N, D, (int64_t)N * D, 1, D, O, D, lse, nullptr, nullptr, stream);
 }
 
 }  // namespace swvr

@@ -36,3 +36,43 @@ def test_dh_split_over_vocabulary_runs(dtype, N, K, V, D, chunk, wrt_h):
         W, E, b = (x.detach() for x in (W, E, b))
     bars = (1e-2, 2e-2) if dtype == torch.bfloat16 else (1e-5, 1e-5)
     check((h, W, E, b), lambda *a: swvr.softmax_readout(*a, chunk_size=chunk), (N,), D, *bars)
+
+
+# the merge of many partial softmaxes in 32 runs (few tokens, a long vocabulary) and in 8 (few
+# partials): rows with every score -inf, whole partials of -inf, and embedding widths off the tiles
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K,V,D", [(1, 40, 70001, 1), (31, 64, 70001, 40), (33, 64, 9000, 33), (700, 64, 2048, 129)])
+def test_merge_of_partials(dtype, N, K, V, D):
+    h, W, E, b = make(N, K, V, D, dtype)
+    with torch.no_grad():
+        b[V // 4:3 * V // 4] = float("-inf")
+    bars = (1e-2, 2e-2) if dtype == torch.bfloat16 else (1e-5, 1e-5)
+    check((h, W, E, b), swvr.softmax_readout, (N,), D, *bars)
+    O, lse = swvr.softmax_readout(h.detach(), W.detach(), E.detach(), torch.full_like(b.detach(), float("-inf")))
+    assert O.isnan().all() and (lse == float("-inf")).all()
+
+
+@pytest.mark.parametrize("N", [1, 1023, 1024, 1025, 4097, 300001])
+def test_compaction_of_active_tokens_over_workgroups(N):
+    """Weights of 0 drop tokens; the others keep their own rows: sizes at the edges of a workgroup's
+    1024 tokens and past 256 workgroups' worth, with a whole workgroup's tokens dropped."""
+    K, V, D = 8, 40, 8
+    h, W, E, b = make(N, K, V, D, torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = (torch.rand(N, generator=g, device="cuda") < 0.4).float()
+    w[2048:3072] = 0
+    t = torch.randn(N, D, generator=g, device="cuda")
+    loss = swvr.softmax_readout_mse(h, W, E, t, b, weight=w, reduction="none")
+    got = torch.autograd.grad(loss.sum(), (h, W))
+    ref = [x.detach().double().requires_grad_(True) for x in (h, W)]
+    O = torch.softmax(ref[0] @ ref[1].T + b.detach().double(), -1) @ E.detach().double()
+    want_loss = (O - t.double()).pow(2).mean(-1) * w.double()
+    want = torch.autograd.grad(want_loss.sum(), ref)
+    if not w.any():
+        assert (loss == 0).all() and all((x == 0).all() for x in got)
+        return
+    # gW sums n terms of either sign in fp32: its partial sums grow like sqrt(k), so the roundings
+    # add up to about sqrt(sum k) 2^-24 against a sum of sqrt(n), sqrt(n / 2) 2^-24; twice that
+    errs = [rel_err(a, r) for a, r in zip((loss, *got), (want_loss, *want))]
+    assert max(errs[:2]) <= 1e-5 and errs[2] <= max(1e-5, w.sum().item() ** 0.5 * 2 ** -23.5), errs
+    assert (got[0][w == 0] == 0).all()
