@@ -105,7 +105,10 @@ int swvr_fwd_mixed(int dtype, int h_dtype, int w_dtype, int64_t N, int64_t K, in
  * (A zero-weight token whose fp32 scores overflow from finite inputs is the one
  * case left: its reference loss is NaN, here 0 * finite.)  O and lse of the
  * computed tokens equal swvr_fwd_mixed's to fp32 rounding (the vocabulary is
- * split differently over the fewer tokens).  No reference counterpart: the
+ * split differently over the fewer tokens).  A call of few tokens (up to 512; fp32
+ * 128) reads W once and computes every token: there a zero-weight token's O
+ * elements and lse are 0 where they are finite, and kept where they are not,
+ * which gives the same loss.  No reference counterpart: the
  * reference computes every token's readout before weighting the loss.
  * Workspace: swvr_fwd_active_workspace_size. */
 size_t swvr_fwd_active_workspace_size(int dtype, int64_t N, int64_t K, int64_t V, int64_t D);

@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256) void pack_vocab_kernel(const T* __restrict__ E
     }
   }
   *reinterpret_cast<V8*>(Ep + e * 8) = x;
-  if (c == 0) {
+  if (c == 0 && biasp) {
     biasp[v] = v < V ? (bias ? bias[v] : 0.f) : kNegInf;
     // e4m3 scores: the factor that turns row v's e4m3 dot product into a score
     if (multp) multp[v] = v < V ? logit_scale * h_scale[0] * w_scale[v] : 0.f;

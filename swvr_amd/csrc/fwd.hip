@@ -685,7 +685,7 @@ template <int G, int DT>
 __global__ __launch_bounds__(G * MergeWidth<G>::value) void fwd_combine_kernel(
     const float* __restrict__ part_m, const float* __restrict__ part_l, const float* __restrict__ part_acc, int n_part,
     int N, int D, int64_t sp, int64_t sd, int64_t sn, float* __restrict__ O, int64_t ldo, float* __restrict__ lse,
-    float* __restrict__ m_out, float* __restrict__ l_out) {
+    float* __restrict__ m_out, float* __restrict__ l_out, const float* __restrict__ weight) {
   constexpr int CW = MergeWidth<G>::value;
   const int64_t e = (int64_t)blockIdx.x * CW + threadIdx.x % CW;
   const int nb = D > 0 ? (D + DT - 1) / DT : 1;
@@ -694,15 +694,20 @@ __global__ __launch_bounds__(G * MergeWidth<G>::value) void fwd_combine_kernel(
   float M, L, a[DT];
   merge_partials<G, DT>(part_m + n, part_l + n, part_acc + d * sd + n * sn, n_part, N, sp, sd, live, D - d, &M, &L, a);
   if (!live || threadIdx.x >= CW) return;
+  const bool zero = weight && weight[n] == 0.f;  // finite values of a zero-weight token: 0
 #pragma unroll
   for (int i = 0; i < DT; ++i)
-    if (d + i < D) O[(int64_t)n * ldo + d + i] = m_out ? a[i] : a[i] / L;
+    if (d + i < D) {
+      const float o = m_out ? a[i] : a[i] / L;
+      O[(int64_t)n * ldo + d + i] = zero && __builtin_isfinite(o) ? 0.f : o;
+    }
   if (d == 0) {
     if (m_out) {
       m_out[n] = M;
       l_out[n] = L;
     } else {
-      lse[n] = M + logf(L);
+      const float x = M + logf(L);
+      lse[n] = zero && __builtin_isfinite(x) ? 0.f : x;
     }
   }
 }
@@ -753,13 +758,13 @@ void dispatch_combine(int64_t elements, int n_part, F&& go) {
 // Merge launch over n_part partials of N rows x D columns (see fwd_combine_kernel).
 hipError_t launch_combine(const float* m, const float* l, const float* acc, int n_part, int N, int D, int64_t sp,
                           int64_t sd, int64_t sn, float* O, int64_t ldo, float* lse, float* m_out, float* l_out,
-                          hipStream_t stream) {
+                          const float* weight, hipStream_t stream) {
   if (N == 0) return hipSuccess;
   timing_begin(kKindFwdCombine, stream);
   auto go = [&](auto g, auto dt) {
     constexpr int G = decltype(g)::value, DT = decltype(dt)::value;
     fwd_combine_kernel<G, DT><<<combine_blocks<G, DT>(N, D), G * MergeWidth<G>::value, 0, stream>>>(
-        m, l, acc, n_part, N, D, sp, sd, sn, O, ldo, lse, m_out, l_out);
+        m, l, acc, n_part, N, D, sp, sd, sn, O, ldo, lse, m_out, l_out, weight);
   };
   dispatch_combine((int64_t)N * D, n_part, go);
   timing_end(kKindFwdCombine, stream);
@@ -924,6 +929,124 @@ hipError_t pack(const FwdParams& p, const FwdPlan& plan, hipStream_t stream) {
 
 }  // namespace
 
+namespace {
+
+// The few-token forward (fwd_few.hip) serves calls of up to this many tokens.  Measured, the whole
+// call in us, general forward -> few-token forward (K, V, D):
+//            N =       64         256         512         1024
+//   bf16 2560, 151936, 64    552 -> 168  569 -> 315   700 -> 570  1080 -> 1062
+//   bf16 1024, 32000, 64     106 -> 54   108 -> 54    114 -> 75    137 -> 120
+//   bf16 4096, 128256, 128   666 -> 228  784 -> 409  1049 -> 748  1471 -> 1414
+//   bf16 768, 50021, 256      91 -> 54   118 -> 96    159 -> 133   271 -> 224
+//   fp32 2560, 32000, 64     333 -> 145  543 -> 401   966 -> 786  1792 -> 1541
+//   autocast 2048, 65536, 128 254 -> 146 269 -> 194   346 -> 308   493 -> 545
+// Past 1024 tokens W is read by enough token blocks for the packing to pay (an fp32 W, whose operands
+// are rounded at every read, sooner).
+constexpr int64_t kFewTokens = 1024, kFewTokensF32W = 768;
+// A weighted loss's forward computes every token here, zero weight or not (the few-token kernel reads
+// W once, so there is no earlier pass that could find its non-finite values), so the line lies where
+// computing all of them costs no more than the general forward of very few active ones.
+constexpr int64_t kFewTokensActive = 512, kFewTokensActiveF32 = 128;
+
+// Tile, split and workspace of the few-token forward for one pass of Dw columns: vocabulary runs
+// so that one workgroup per CU covers the vocabulary, whole 32-row groups each.
+void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, FwdPlan* plan) {
+  plan->few = dtype != kFP8 && N <= (!active ? kFewTokens : dtype == kF32 ? kFewTokensActiveF32 : kFewTokensActive);
+  if (!plan->few) return;
+  const bool two = dtype != kF32;
+  plan->few_DP = Dw <= 64 ? 64 : Dw <= 128 ? 128 : 256;
+  const int nb_max = two && plan->few_DP <= 128 ? 4 : 2;
+  plan->few_NB = N <= 32 ? 1 : N <= 64 || nb_max == 2 ? 2 : 4;
+  plan->few_tb = (int)((N + 32 * plan->few_NB - 1) / (32 * plan->few_NB));
+  const int64_t grp = (V + 31) / 32, cu = 256 / (plan->few_tb > 0 ? plan->few_tb : 1);
+  plan->few_split = (int)(grp < 1 ? 1 : grp < cu ? grp : cu);
+  const size_t part = (size_t)plan->few_split * N * 4;
+  const size_t tb = two ? 2 : 4;
+  const int sk = two ? SliceK<bf16_t>::value : SliceK<float>::value;
+  size_t off = 0;
+  plan->few_m = off;
+  off += align256(part);
+  plan->few_l = off;
+  off += align256(part);
+  plan->few_acc = off;
+  off += align256(part * plan->few_DP);
+  plan->few_hp = off;
+  off += align256((size_t)plan->N_pad * plan->hS * sk * tb);
+  plan->few_E = off;  // aligned copy of E's rows, for a caller's E that is not
+  off += align256((size_t)plan->V_pad * plan->few_DP * tb);
+  if (off > plan->ws_bytes) plan->ws_bytes = off;
+}
+
+// Whether the call takes the few-token forward: an fp32 W's line, and 32-bit offsets that reach 128
+// rows of W and E.
+bool few_fits(const FwdPlan& plan, const FwdParams& p, int dtype) {
+  const int64_t esz = dtype == kF32 ? 4 : 2, wsz = p.w_f32 ? 4 : esz, lim = (int64_t)1 << 31;
+  return plan.few && (!p.w_f32 || p.N <= kFewTokensF32W) && p.ldw * wsz * 128 < lim && p.lde * esz * 128 < lim;
+}
+
+// With weight set (a weighted loss), a finite O element or LSE of a zero-weight token is written as 0.
+template <class T>
+hipError_t fwd_few_typed(int dtype, const FwdPlan& plan, const FwdParams& p, const float* weight, char* ws, float* O,
+                         float* lse, float* m_out, float* l_out, hipStream_t stream) {
+  T* const hp = reinterpret_cast<T*>(ws + plan.few_hp);
+  FwdFewParams q{};
+  q.hp = hp;
+  q.hS = plan.hS;
+  q.W = p.W;
+  q.ldw = p.ldw;
+  q.w_f32 = p.w_f32;
+  q.bias = p.bias;
+  q.scale = p.scale;
+  q.N = p.N;
+  q.K = p.K;
+  q.V = p.V;
+  q.DP = plan.few_DP;
+  q.NB = plan.few_NB;
+  q.n_tb = plan.few_tb;
+  q.n_split = plan.few_split;
+  q.part_m = reinterpret_cast<float*>(ws + plan.few_m);
+  q.part_l = reinterpret_cast<float*>(ws + plan.few_l);
+  q.part_acc = reinterpret_cast<float*>(ws + plan.few_acc);
+  timing_begin(kKindPack, stream);
+  hipError_t e = pack_src<T>(p.h, p.h_f32, p.ldh, p.N, p.K, plan.hS, plan.N_pad, hp, stream);
+  timing_end(kKindPack, stream);
+  for (int d0 = 0; e == hipSuccess && d0 < (p.D > 0 ? p.D : 1); d0 += plan.DS) {
+    const T* E = static_cast<const T*>(p.E) + d0;
+    q.D = p.D - d0 < plan.DS ? p.D - d0 : plan.DS;
+    q.E = E;
+    q.lde = p.lde;
+    if (p.V > 0 && q.D > 0 && !(rows_vec16(E, p.lde) && q.D % (16 / (int)sizeof(T)) == 0)) {
+      // E's rows as 16-byte chunks, zero past D
+      T* const Ep = reinterpret_cast<T*>(ws + plan.few_E);
+      const int64_t n = (int64_t)p.V * (plan.few_DP / 8);
+      timing_begin(kKindPack, stream);
+      pack_vocab_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(
+          E, p.lde, nullptr, p.V, q.D, p.V, plan.few_DP, rows_vec16(E, p.lde), Ep, nullptr);
+      timing_end(kKindPack, stream);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+      q.E = Ep;
+      q.lde = plan.few_DP;
+      q.D = plan.few_DP;
+    }
+    if ((e = fwd_few_launch(dtype, q, stream)) != hipSuccess) return e;
+    const int D = p.D - d0 < plan.DS ? p.D - d0 : plan.DS;
+    e = launch_combine(q.part_m, q.part_l, q.part_acc, q.n_split, p.N, D, (int64_t)plan.few_DP * p.N, p.N, 1,
+                       O ? O + d0 : nullptr, p.D, lse, m_out, l_out, weight, stream);
+  }
+  return e;
+}
+
+hipError_t fwd_few(int dtype, const FwdPlan& plan, const FwdParams& p, const float* weight, char* ws, float* O,
+                   float* lse, float* m_out, float* l_out, hipStream_t stream) {
+  switch (dtype) {
+    case kBF16: return fwd_few_typed<bf16_t>(dtype, plan, p, weight, ws, O, lse, m_out, l_out, stream);
+    case kF16: return fwd_few_typed<f16_t>(dtype, plan, p, weight, ws, O, lse, m_out, l_out, stream);
+    default: return fwd_few_typed<float>(dtype, plan, p, weight, ws, O, lse, m_out, l_out, stream);
+  }
+}
+
+}  // namespace
+
 bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* plan, bool active) {
   (void)K;
   if (active && dtype == kFP8) return false;
@@ -1007,12 +1130,14 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
     off += 256;
   }
   plan->ws_bytes = off;
+  few_plan(dtype, N, V, Dw, active, plan);
   return true;
 }
 
 hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, float* O, float* lse, float* m_out,
                       float* l_out, hipStream_t stream) {
   if (p.N == 0) return hipSuccess;
+  if (few_fits(plan, p, dtype)) return fwd_few(dtype, plan, p, nullptr, ws, O, lse, m_out, l_out, stream);
   p.n_tb = plan.n_tb;
   p.n_split = plan.n_split;
   p.n_vt = plan.n_vt;
@@ -1049,7 +1174,7 @@ hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, flo
     if (e != hipSuccess) return e;
     // every pass computes the same scores, so each writes the same lse (m, l); O gets its columns
     e = launch_combine(p.part_m, p.part_l, p.part_acc, plan.n_part, p.N, q.D, (int64_t)plan.DP * p.N, p.N, 1,
-                       O ? O + d0 : nullptr, D, lse, m_out, l_out, stream);
+                       O ? O + d0 : nullptr, D, lse, m_out, l_out, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1111,6 +1236,7 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
                              float* lse, hipStream_t stream) {
   if (p.N == 0) return hipSuccess;
   if (!plan.active || dtype == kFP8) return hipErrorInvalidValue;
+  if (few_fits(plan, p, dtype)) return fwd_few(dtype, plan, p, weight, ws, O, lse, nullptr, nullptr, stream);
   p.n_tb = plan.n_tb;
   p.n_split = plan.n_split;
   p.n_vt = plan.n_vt;
@@ -1162,7 +1288,8 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
 
 hipError_t shard_combine(int S, int N, int D, const float* m, const float* l, const float* acc, float* O, float* lse,
                          hipStream_t stream) {
-  return launch_combine(m, l, acc, S, N, D, (int64_t)N * D, 1, D, O, D, lse, nullptr, nullptr, stream);
+  return launch_combine(m, l, acc, S, N, D, (int64_t)N * D, 1, D, O, D, lse, nullptr, nullptr, nullptr,
+                        stream);
 }
 
 }  // namespace swvr

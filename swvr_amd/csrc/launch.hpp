@@ -103,6 +103,10 @@ struct FwdPlan {
   bool active;
   int WV;
   size_t off_flag, off_idx, off_inv, off_nact;
+  // few tokens (fwd_few.hip): tile, split and workspace of that path; few = false: not taken
+  bool few;
+  int few_DP, few_NB, few_tb, few_split;
+  size_t few_m, few_l, few_acc, few_hp, few_E;
 };
 
 // fwd_plan / fwd_launch dtype of the e4m3 forward (h, W in e4m3; E in bf16).
@@ -119,9 +123,30 @@ hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, flo
 // and lse of the others are 0.  A zero-weight token whose h row holds an
 // infinity or a NaN stays active, and so does every token when W, E or the
 // bias holds a NaN or +inf or when every bias entry is -inf: the rows whose
-// loss the reference makes NaN (0 * NaN) are computed.  Plan with active set.
+// loss the reference makes NaN (0 * NaN) are computed.  With few tokens every token is computed, and
+// the finite values of a zero-weight one written as 0.  Plan with active set.
 hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const float* weight, char* ws, float* O,
                              float* lse, hipStream_t stream);
+// ---- few tokens (fwd_few.hip): W and E read as the caller stores them
+struct FwdFewParams {
+  const void* hp;      // h packed in its tiles' LDS image (pack_rows_tiled_kernel), hS slices
+  int hS;
+  const void* W;       // [V][ldw]: the compute dtype, or fp32 (w_f32) under a 2-byte one
+  int64_t ldw;
+  int w_f32;
+  const void* E;       // [V][lde], 16-byte aligned rows of D columns, D a multiple of the 16-byte chunk
+  int64_t lde;
+  const float* bias;   // [V] or null
+  float scale;
+  int N, K, V, D;
+  int DP, NB;          // padded D (64, 128, 256), 32-token blocks per workgroup (1, 2, 4)
+  int n_tb, n_split;   // token blocks, vocabulary runs
+  float* part_m;       // [n_split][N]
+  float* part_l;
+  float* part_acc;     // [n_split][DP][N]
+};
+hipError_t fwd_few_launch(int dtype, const FwdFewParams& p, hipStream_t stream);
+
 // Order-preserving compaction of flagged tokens (flag[n] != 0): idx[q] = token
 // of position q, inv[n] = position of token n or -1, n_act[0] = count.
 hipError_t compact_tokens(const int* flag, int N, int* idx, int* inv, int* n_act, hipStream_t stream);

@@ -76,3 +76,80 @@ def test_compaction_of_active_tokens_over_workgroups(N):
     errs = [rel_err(a, r) for a, r in zip((loss, *got), (want_loss, *want))]
     assert max(errs[:2]) <= 1e-5 and errs[2] <= max(1e-5, w.sum().item() ** 0.5 * 2 ** -23.5), errs
     assert (got[0][w == 0] == 0).all()
+
+
+# the few-token forward: every token-block width, embedding width and storage type of it, sizes at the
+# edges of its 32-token blocks, 128-row tiles, 128-byte slices and ring (short reductions), vocabularies
+# of less than a group and of ragged runs, embeddings that need an aligned copy, several passes of columns
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32", "autocast"])
+@pytest.mark.parametrize("N,K,V,D", [
+    (1, 72, 20011, 64), (31, 8, 97, 8), (32, 512, 9001, 200), (33, 40, 31, 128), (64, 1032, 5000, 33),
+    (65, 264, 16385, 64), (128, 100, 4097, 72), (129, 96, 8193, 256), (255, 2048, 600, 300), (256, 64, 1, 16),
+    (769, 64, 900, 64), (1024, 136, 2000, 130),
+])
+def test_few_token_forward(dtype, N, K, V, D):
+    amp = dtype == "autocast"
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16}.get(dtype, torch.float32)
+    h, W, E, b = make(N, K, V, D, dt, requires_grad=False)
+    b[1:V // 3] = float("-inf")
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+        O, lse = swvr.softmax_readout(h, W, E, b, logit_scale=0.7)
+    cd = torch.bfloat16 if amp else dt
+    hd, Wd, Ed = (x.to(cd).double() for x in (h, W, E))
+    S = 0.7 * (hd @ Wd.T) + b.double()
+    want_O, want_lse = torch.softmax(S, -1) @ Ed, torch.logsumexp(S, -1)
+    bar = 1e-5 if cd == torch.float32 else 1e-2
+    assert rel_err(O, want_O) <= bar and rel_err(lse, want_lse) <= bar, (rel_err(O, want_O), rel_err(lse, want_lse))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_few_token_forward_equals_the_general_one_over_strides(dtype):
+    """Strided h, W and E (row strides beyond their width, columns starting off 16 bytes) and a shard's
+    partials: the same readout as from dense operands, and as rows of a call of many tokens."""
+    from swvr_amd import vocab_shard as vs
+    N, K, V, D = 40, 96, 3001, 48
+    g = torch.Generator(device="cuda").manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    h, W, E, b = r(300, K + 24)[:, 8:8 + K], r(V, K + 40)[:, 16:16 + K] / 8, r(V, D + 3)[:, 1:1 + D], r(V).float()
+    O, lse = swvr.softmax_readout(h[:N], W, E, b)
+    O_all, lse_all = swvr.softmax_readout(h, W, E, b)
+    O_dense, lse_dense = swvr.softmax_readout(h[:N].contiguous(), W.contiguous(), E.contiguous(), b)
+    assert torch.equal(O, O_dense) and torch.equal(lse, lse_dense)
+    bar = 1e-5 if dtype == torch.float32 else 2e-3
+    assert rel_err(O, O_all[:N]) <= bar and rel_err(lse, lse_all[:N]) <= 1e-5
+    parts = [vs.softmax_readout_partial(h[:N], W[s], E[s], b[s]) for s in (slice(0, 1000), slice(1000, V))]
+    O_s, lse_s = vs.combine_partials(*(torch.stack(x) for x in zip(*parts)))
+    assert rel_err(O_s, O) <= bar and rel_err(lse_s, lse) <= 1e-5
+
+
+def test_few_token_forward_keeps_non_finite_rows_apart():
+    """An infinity or NaN in one token's h reaches that token alone, also where K ends inside a slice
+    (the padding of h and W multiply to zero) and where the block holds other tokens."""
+    N, K, V, D = 20, 40, 500, 16
+    h, W, E, b = make(N, K, V, D, torch.bfloat16, requires_grad=False)
+    h[3, 7], h[11, 39] = float("inf"), float("nan")
+    O, lse = swvr.softmax_readout(h, W, E, b)
+    bad = torch.zeros(N, dtype=torch.bool, device="cuda")
+    bad[[3, 11]] = True
+    assert O[bad].isnan().all() and O[~bad].isfinite().all() and lse[~bad].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [1, 128, 129, 512, 513])
+def test_weighted_few_token_forward_zeroes_the_rows_of_zero_weight(dtype, N):
+    """Both sides of the lines to the general active-token forward (128 in fp32, 512 else): the rows of
+    non-zero weight as the unweighted call has them, zero rows for the others, a NaN column of E kept."""
+    from swvr_amd import _ops
+    K, V, D = 64, 700, 24
+    h, W, E, b = make(N, K, V, D, dtype)
+    w = (torch.arange(N, device="cuda") % 3 != 1).float()
+    with torch.no_grad():
+        O, lse = _ops._forward_active(h, W, E, b, w, 1.0, 8192, dtype)
+        full = swvr.softmax_readout(h, W, E, b)
+    on, bar = w != 0, 1e-5 if dtype == torch.float32 else 2e-3
+    assert (O[~on] == 0).all() and (lse[~on] == 0).all()
+    assert rel_err(O[on], full[0][on]) <= bar and rel_err(lse[on], full[1][on]) <= 1e-5
+    bad = E.detach().clone()
+    bad[V // 2, 3] = float("nan")
+    O, lse = _ops._forward_active(h.detach(), W.detach(), bad, b.detach(), w, 1.0, 8192, dtype)
+    assert O[:, 3].isnan().all() and (lse[on] != 0).all()
