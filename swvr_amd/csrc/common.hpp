@@ -70,6 +70,10 @@ __device__ __forceinline__ f32x16_t zero16() {
 // exp(x) as 2^(x*log2 e) on the hardware exp2 (v_exp_f32).  exp(-inf) = 0.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
+// Shift of P = e^(s - shift) in the forwards: a vocabulary tile's own maximum, but at most this far
+// below the running one (which bounds P's sums).
+constexpr float kShiftBelow = 8.f;
+
 template <class T> __device__ __forceinline__ T from_float(float x) { return (T)x; }
 template <class T> __device__ __forceinline__ float to_float(T x) { return (float)x; }
 

@@ -18,6 +18,11 @@
 //     (an independent partial softmax), and P, rounded to the compute dtype as
 //     the reference rounds it (swvr/chunked.py:103, triton_kernels.py:69),
 //     feeds acc^T += E^T P^T straight from the score registers;
+//     P is relative to the tile's own maximum (within 8 of the running one), not
+//     the running maximum: the maximum's row has P = 1, which no rounding
+//     changes, so most rows that dominate a peaked softmax stay exact (O of 3000
+//     tokens on V = 151936 at a logit spread of 3: 1.0e-4 from 64 bits in bf16,
+//     1.7e-4 with the running maximum), whatever the number of splits;
 //   * partials (m, l, acc) of all waves and splits are merged by
 //     fwd_combine_kernel in a fixed order (deterministic).
 #include <cmath>
@@ -171,11 +176,11 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
   const int vt_end = (int)((int64_t)(split + 1) * p.n_vt / n_split);
   const T* Ep = static_cast<const T*>(p.Ep);
 
-  float m[FT], l[FT];
+  float m[FT], sh[FT], l[FT];  // running maximum, the shift l and acc are relative to
   f32x16_t oacc[DB][FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
-    m[ft] = kNegInf;
+    m[ft] = sh[ft] = kNegInf;
     l[ft] = 0.f;
 #pragma unroll
     for (int db = 0; db < DB; ++db) oacc[db][ft] = zero16();
@@ -269,12 +274,16 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
       }
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
-      const float mnew = fmaxf(m[ft], wave_max32(mx[ft]));
-      // a column whose scores so far are all -inf keeps m = -inf; shift it by 0
+      const float mt = wave_max32(mx[ft]), mnew = fmaxf(m[ft], mt);
+      // the e4m3 forward, whose operands are rounded far more coarsely, keeps the running maximum
+      // (0.8% faster there)
+      const float snew = F8 ? mnew : fmaxf(mt, mnew - kShiftBelow);
+      // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
-      const float shift = mnew == kNegInf ? 0.f : mnew;
-      const float alpha = fast_exp(m[ft] - shift);
+      const float shift = snew == kNegInf ? 0.f : snew;
+      const float alpha = fast_exp((F8 ? m[ft] : sh[ft]) - shift);  // at most e^kShiftBelow
       m[ft] = mnew;
+      if (!F8) sh[ft] = snew;
       float rs = 0.f;
 #pragma unroll
       for (int fv = 0; fv < FV; ++fv)
@@ -333,17 +342,19 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
     const int n = n0 + wt * WTR + ft * 32 + (ln & 31);
+    // to the running maximum; no score yet: 0
+    const float f = F8 ? 1.f : m[ft] == kNegInf ? 0.f : fast_exp(sh[ft] - m[ft]);
     if (n < ntok) {
       if (ln < 32) {
         p.part_m[(int64_t)part * ntok + n] = m[ft];
-        p.part_l[(int64_t)part * ntok + n] = l[ft];
+        p.part_l[(int64_t)part * ntok + n] = l[ft] * f;
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int d = db * 32 + c_row(r, ln);
-          p.part_acc[((int64_t)part * DP + d) * ntok + n] = oacc[db][ft][r];
+          p.part_acc[((int64_t)part * DP + d) * ntok + n] = oacc[db][ft][r] * f;
         }
     }
   }
@@ -403,11 +414,11 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
   const int vt_end = (int)((int64_t)(split + 1) * p.n_vt / n_split);
   const T* Ep = static_cast<const T*>(p.Ep);
 
-  float m[FT], l[FT];
+  float m[FT], sh[FT], l[FT];  // running maximum, the shift l and acc are relative to
   f32x16_t oacc[DB][FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
-    m[ft] = kNegInf;
+    m[ft] = sh[ft] = kNegInf;
     l[ft] = 0.f;
 #pragma unroll
     for (int db = 0; db < DB; ++db) oacc[db][ft] = zero16();
@@ -515,12 +526,14 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
       }
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
-      const float mnew = fmaxf(m[ft], wave_max32(mx[ft]));
-      // a column whose scores so far are all -inf keeps m = -inf; shift it by 0
+      const float mt = wave_max32(mx[ft]);
+      m[ft] = fmaxf(m[ft], mt);
+      const float snew = fmaxf(mt, m[ft] - kShiftBelow);
+      // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
-      const float shift = mnew == kNegInf ? 0.f : mnew;
-      const float alpha = fast_exp(m[ft] - shift);
-      m[ft] = mnew;
+      const float shift = snew == kNegInf ? 0.f : snew;
+      const float alpha = fast_exp(sh[ft] - shift);  // at most e^kShiftBelow
+      sh[ft] = snew;
       float rs = 0.f;
 #pragma unroll
       for (int fv = 0; fv < FV; ++fv)
@@ -573,17 +586,18 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
     const int n = n0 + wt * WTR + ft * 32 + (ln & 31);
+    const float f = m[ft] == kNegInf ? 0.f : fast_exp(sh[ft] - m[ft]);  // to the running maximum; no score yet: 0
     if (n < ntok) {
       if (ln < 32) {
         p.part_m[(int64_t)part * ntok + n] = m[ft];
-        p.part_l[(int64_t)part * ntok + n] = l[ft];
+        p.part_l[(int64_t)part * ntok + n] = l[ft] * f;
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int d = db * 32 + c_row(r, ln);
-          p.part_acc[((int64_t)part * DP + d) * ntok + n] = oacc[db][ft][r];
+          p.part_acc[((int64_t)part * DP + d) * ntok + n] = oacc[db][ft][r] * f;
         }
     }
   }
@@ -931,6 +945,30 @@ hipError_t pack(const FwdParams& p, const FwdPlan& plan, hipStream_t stream) {
 
 namespace {
 
+// Vocabulary splits of a forward whose workgroups hold a CU each, from the rule's n_split: the split
+// that ends soonest when n_tb x s workgroups run 256 at a time, if it is 3% sooner.  A workgroup takes
+// n_vt / s vocabulary tiles on average ((K + DP) / 32 slices of 0.3 us per 128 tokens each) and about 5 us
+// of ring fill and partial stores; a single round ends with its longest, several even out half of that.
+// 2500 tokens on V = 50021, K = 768, D = 256 (20 token blocks): 52 splits are 1040 workgroups, a fifth
+// round for 16 of them, and the pass took 436 us; 25 make 2 whole rounds, 356 us.
+int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int64_t K, int DP, int BM) {
+  const double tile = ((double)K + DP) / 32 * 0.3 * (BM / 128.0), over = 5.0;
+  auto span = [&](int64_t s) {
+    const int64_t rounds = (n_tb * s + kFwdRound - 1) / kFwdRound;
+    const double avg = (double)n_vt / s, rest = (double)((n_vt + s - 1) / s) - avg;
+    return rounds * (avg * tile + over) + rest * tile * (rounds > 1 ? 0.5 : 1.0);
+  };
+  double best = 0.97 * span(n_split);
+  const int64_t cap = n_vt / 2 > 1 ? n_vt / 2 : 1, hi = 4 * (int64_t)kFwdRound / n_tb;
+  int pick = n_split;
+  for (int64_t s = 1; s <= hi && s <= cap; ++s)
+    if (span(s) < best) {
+      best = span(s);
+      pick = (int)s;
+    }
+  return pick;
+}
+
 // The few-token forward (fwd_few.hip) serves calls of up to this many tokens.  Measured, the whole
 // call in us, general forward -> few-token forward (K, V, D):
 //            N =       64         256         512         1024
@@ -1094,20 +1132,37 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
     const int max_split = plan->n_vt / 2 > 1 ? plan->n_vt / 2 : 1;
     if (n_split > max_split) n_split = max_split;
     if (n_split < 1) n_split = 1;
+    if (!active && tbytes == 2 && dtype != kFP8) n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, K, DP, BM);
   }
   plan->n_split = n_split;
   plan->n_part = WV * n_split;
   plan->WV = WV;
+  plan->rem_DP = 0;
+  int64_t parts = plan->n_part;  // partials, and partials x columns, the buffers hold: the larger of the passes'
+  int64_t part_cols = (int64_t)plan->n_part * DP;
+  if (!active && plan->n_dslices > 1 && N > 0) {
+    FwdPlan rem;
+    fwd_plan(dtype, N, K, V, D - (int64_t)(plan->n_dslices - 1) * DS, &rem);
+    if (rem.DP < DP && rem.BV == BV) {
+      plan->rem_DP = rem.DP;
+      plan->rem_BM = rem.BM;
+      plan->rem_tb = rem.n_tb;
+      plan->rem_split = rem.n_split;
+      plan->rem_part = rem.n_part;
+      if (rem.n_part > parts) parts = rem.n_part;
+      if ((int64_t)rem.n_part * rem.DP > part_cols) part_cols = (int64_t)rem.n_part * rem.DP;
+    }
+  }
   // token rows of a partial: N; the active-token forward's partials hold up to
   // 2 x n_tb x n_split workgroups' n_tb x BM positions each (active_grid)
   const int64_t NR = active ? 2 * (int64_t)plan->n_tb * BM : N;
   size_t off = 0;
   plan->off_m = off;
-  off += align256((size_t)plan->n_part * NR * 4);
+  off += align256((size_t)parts * NR * 4);
   plan->off_l = off;
-  off += align256((size_t)plan->n_part * NR * 4);
+  off += align256((size_t)parts * NR * 4);
   plan->off_acc = off;
-  off += align256((size_t)plan->n_part * NR * 4 * DP);
+  off += align256((size_t)part_cols * NR * 4);
   plan->off_Ep = off;
   off += align256((size_t)plan->V_pad * DP * tbytes);
   plan->off_bias = off;
@@ -1165,15 +1220,23 @@ hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, flo
     FwdParams q = p;
     q.E = static_cast<const char*>(p.E) + d0 * esz;
     q.D = D - d0 < plan.DS ? D - d0 : plan.DS;
+    FwdPlan pass = plan;
+    if (plan.rem_DP > 0 && d0 + plan.DS >= D) {  // the last, narrower pass: its own kernel, tiles and split
+      pass.DP = plan.rem_DP;
+      pass.BM = plan.rem_BM;
+      pass.n_tb = q.n_tb = plan.rem_tb;
+      pass.n_split = q.n_split = plan.rem_split;
+      pass.n_part = plan.rem_part;
+    }
     switch (dtype) {
-      case kBF16: e = pack_et<bf16_t>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<bf16_t>(plan, q, stream); break;
-      case kF16: e = pack_et<f16_t>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<f16_t>(plan, q, stream); break;
-      case kF32: e = pack_et<float>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<float>(plan, q, stream); break;
-      default: e = pack_et<bf16_t>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp_f8(plan, q, stream); break;
+      case kBF16: e = pack_et<bf16_t>(q, pass, stream); if (e == hipSuccess) e = dispatch_dp<bf16_t>(pass, q, stream); break;
+      case kF16: e = pack_et<f16_t>(q, pass, stream); if (e == hipSuccess) e = dispatch_dp<f16_t>(pass, q, stream); break;
+      case kF32: e = pack_et<float>(q, pass, stream); if (e == hipSuccess) e = dispatch_dp<float>(pass, q, stream); break;
+      default: e = pack_et<bf16_t>(q, pass, stream); if (e == hipSuccess) e = dispatch_dp_f8(pass, q, stream); break;
     }
     if (e != hipSuccess) return e;
     // every pass computes the same scores, so each writes the same lse (m, l); O gets its columns
-    e = launch_combine(p.part_m, p.part_l, p.part_acc, plan.n_part, p.N, q.D, (int64_t)plan.DP * p.N, p.N, 1,
+    e = launch_combine(p.part_m, p.part_l, p.part_acc, pass.n_part, p.N, q.D, (int64_t)pass.DP * p.N, p.N, 1,
                        O ? O + d0 : nullptr, D, lse, m_out, l_out, nullptr, stream);
     if (e != hipSuccess) return e;
   }

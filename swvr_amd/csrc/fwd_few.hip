@@ -14,8 +14,11 @@
 //   * W arrives in 128-byte row pieces through an LDS ring as deep as the 160 KB
 //     allow, so 48 to 100 KB of W are in flight per CU: the loop is bound by HBM.
 //     Rows past the run are not loaded;
-//   * the online softmax and acc^T += E^T P^T run as in the general forward; the
-//     E^T operand is read from the row-major E tile with transposing LDS reads;
+//   * the online softmax and acc^T += E^T P^T run as in the general forward,
+//     the tile of 128 rows being each wave's own 32: its maximum, which P's
+//     rounding leaves exact, is the shift of P (O of 1000 tokens on V = 151936 at a
+//     logit spread of 3: 5.8e-5 from 64 bits in bf16, 1.3e-4 with running maxima).
+//     The E^T operand is read from the row-major E tile with transposing LDS reads;
 //   * the waves' partial softmaxes are merged in LDS, so a workgroup writes one
 //     partial; fwd_combine_kernel merges those in a fixed order.
 #include <type_traits>
@@ -103,8 +106,8 @@ struct FewCfg {
   static constexpr int NS = FIT < 8 ? FIT : 8;
   static_assert(NS >= 3 && (NS - 2) * L < 64, "ring depth");
   static constexpr int LDS = NS * SB + TE::BYTES;
-  // the merge of the waves' partials reuses the LDS: 4 x [DP][32] floats, then 4 x [32 NB] m and l
-  static_assert(kFewWV * (DP * 32 + 2 * 32 * NB) * 4 <= LDS, "merge fits");
+  // the merge of the waves' partials reuses the LDS: 4 x [DP][32] floats, then 4 x [32 NB] of three
+  static_assert(kFewWV * (DP * 32 + 3 * 32 * NB) * 4 <= LDS, "merge fits");
 };
 
 // At most min(ahead, MAX) stages of L loads may stay outstanding.
@@ -187,11 +190,12 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue_next();
 
-  float m[FT], l[FT];
+  // running maximum, and the shift that l and acc are relative to
+  float m[FT], sh[FT], l[FT];
   f32x16_t oacc[DB][FT], sacc[FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
-    m[ft] = kNegInf;
+    m[ft] = sh[ft] = kNegInf;
     l[ft] = 0.f;
 #pragma unroll
     for (int db = 0; db < DB; ++db) oacc[db][ft] = zero16();
@@ -260,12 +264,14 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
         sacc[ft][r] = x;
         mx = fmaxf(mx, x);
       }
-      const float mnew = fmaxf(m[ft], wave_max32(mx));
-      // a column whose scores so far are all -inf keeps m = -inf; shift it by 0
+      mx = wave_max32(mx);
+      m[ft] = fmaxf(m[ft], mx);
+      const float snew = fmaxf(mx, m[ft] - kShiftBelow);
+      // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
-      const float shift = mnew == kNegInf ? 0.f : mnew;
-      const float alpha = fast_exp(m[ft] - shift);
-      m[ft] = mnew;
+      const float shift = snew == kNegInf ? 0.f : snew;
+      const float alpha = fast_exp(sh[ft] - shift);  // at most e^kShiftBelow
+      sh[ft] = snew;
       float rs = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -303,12 +309,14 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
   float* const sA = reinterpret_cast<float*>(smem);  // [4][DP][32]
   float* const sM = sA + kFewWV * DP * 32;           // [4][32 NB]
   float* const sL = sM + kFewWV * 32 * NB;           // [4][32 NB]
+  float* const sS = sL + kFewWV * 32 * NB;           // [4][32 NB]
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft)
     if (lane < 32) {
       const int c = (wt * FT + ft) * 32 + lane;
       sM[wv * 32 * NB + c] = m[ft];
       sL[wv * 32 * NB + c] = l[ft];
+      sS[wv * 32 * NB + c] = sh[ft];
     }
   __syncthreads();
   for (int bt = 0; bt < WT; ++bt)
@@ -320,7 +328,7 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       for (int j = 0; j < kFewWV; ++j) M = fmaxf(M, sM[j * 32 * NB + c]);
       const float shift = M == kNegInf ? 0.f : M;
       if (wt == bt) {
-        const float f = fast_exp(m[ft] - shift);  // exp(-inf) = 0: a wave of masked rows adds nothing
+        const float f = fast_exp(sh[ft] - shift);  // exp(-inf) = 0: a wave of masked rows adds nothing
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -336,7 +344,7 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       if (w == 0 && lane < 32 && n0 + c < p.N) {
         float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < kFewWV; ++j) sum += sL[j * 32 * NB + c] * fast_exp(sM[j * 32 * NB + c] - shift);
+        for (int j = 0; j < kFewWV; ++j) sum += sL[j * 32 * NB + c] * fast_exp(sS[j * 32 * NB + c] - shift);
         p.part_m[(int64_t)split * p.N + n0 + c] = M;
         p.part_l[(int64_t)split * p.N + n0 + c] = sum;
       }

@@ -103,6 +103,8 @@ struct FwdPlan {
   bool active;
   int WV;
   size_t off_flag, off_idx, off_inv, off_nact;
+  // the last pass of a D in several passes, when it is narrow enough for a narrower kernel (rem_DP > 0)
+  int rem_DP, rem_BM, rem_tb, rem_split, rem_part;
   // few tokens (fwd_few.hip): tile, split and workspace of that path; few = false: not taken
   bool few;
   int few_DP, few_NB, few_tb, few_split;

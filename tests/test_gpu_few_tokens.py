@@ -153,3 +153,18 @@ def test_weighted_few_token_forward_zeroes_the_rows_of_zero_weight(dtype, N):
     bad[V // 2, 3] = float("nan")
     O, lse = _ops._forward_active(h.detach(), W.detach(), bad, b.detach(), w, 1.0, 8192, dtype)
     assert O[:, 3].isnan().all() and (lse[on] != 0).all()
+
+
+# embeddings wider than one pass whose last pass runs on a narrower kernel (64, 128 columns, whole
+# passes beside), with token counts whose vocabulary splits are balanced and ones where they are not
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("N,K,V,D", [(2500, 64, 9000, 300), (1100, 96, 3000, 257), (3000, 40, 4097, 640),
+                                     (1030, 64, 300, 384)])
+def test_last_pass_of_wide_embeddings_on_a_narrower_kernel(dtype, N, K, V, D):
+    h, W, E, b = make(N, K, V, D, dtype, requires_grad=False)
+    O, lse = swvr.softmax_readout(h, W, E, b)
+    S = h.double() @ W.double().T + b.double()
+    bar = 1e-5 if dtype == torch.float32 else 1e-2
+    for sl in (slice(0, D // 256 * 256), slice(D // 256 * 256, D)):
+        assert sl.start == sl.stop or rel_err(O[:, sl], torch.softmax(S, -1) @ E.double()[:, sl]) <= bar
+    assert rel_err(lse, torch.logsumexp(S, -1)) <= bar
