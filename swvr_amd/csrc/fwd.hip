@@ -978,30 +978,36 @@ int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int64_t K, int DP, i
 //   bf16 768, 50021, 256      91 -> 54   118 -> 96    159 -> 133   271 -> 224
 //   fp32 2560, 32000, 64     333 -> 145  543 -> 401   966 -> 786  1792 -> 1541
 //   autocast 2048, 65536, 128 254 -> 146 269 -> 194   346 -> 308   493 -> 545
-// Past 1024 tokens W is read by enough token blocks for the packing to pay (an fp32 W, whose operands
-// are rounded at every read, sooner).
-constexpr int64_t kFewTokens = 1024, kFewTokensF32W = 768;
-// A weighted loss's forward computes every token here, zero weight or not (the few-token kernel reads
-// W once, so there is no earlier pass that could find its non-finite values), so the line lies where
-// computing all of them costs no more than the general forward of very few active ones.
+// Towards 1024 tokens W is read by enough token blocks for the packing to pay, under autocast before
+// that (an fp32 W's operands are rounded at every read); one line for both, so that an fp32 W gives the
+// bits of one cast beforehand.  fp32 calls take it at any size (8192 tokens: 13.3 -> 10.7 ms).
+constexpr int64_t kFewTokens = 768;
+// A weighted loss's forward of up to this many tokens computes all of them, zero weight or not: the
+// one pass over W costs no more than the passes that find the active ones do with W to be searched for
+// non-finite values first.  Past it the few-token kernel runs over the active tokens' positions.
 constexpr int64_t kFewTokensActive = 512, kFewTokensActiveF32 = 128;
 
-// Tile, split and workspace of the few-token forward for one pass of Dw columns: vocabulary runs
-// so that one workgroup per CU covers the vocabulary, whole 32-row groups each.
-void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, FwdPlan* plan) {
-  plan->few = dtype != kFP8 && N <= (!active ? kFewTokens : dtype == kF32 ? kFewTokensActiveF32 : kFewTokensActive);
+// Tile, split and workspace (from offset off on) of the few-token forward for one pass of Dw columns:
+// vocabulary runs of whole 32-row groups.
+void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, size_t off, FwdPlan* plan) {
+  plan->few = dtype != kFP8 && (dtype == kF32 || N <= kFewTokens);
   if (!plan->few) return;
   const bool two = dtype != kF32;
-  plan->few_DP = Dw <= 64 ? 64 : Dw <= 128 ? 128 : 256;
-  const int nb_max = two && plan->few_DP <= 128 ? 4 : 2;
+  plan->few_DP = !two && Dw <= 32 ? 32 : Dw <= 64 ? 64 : Dw <= 128 ? 128 : 256;
+  const int nb_max = plan->few_DP <= 128 ? 4 : 2;
   plan->few_NB = N <= 32 ? 1 : N <= 64 || nb_max == 2 ? 2 : 4;
   plan->few_tb = (int)((N + 32 * plan->few_NB - 1) / (32 * plan->few_NB));
-  const int64_t grp = (V + 31) / 32, cu = 256 / (plan->few_tb > 0 ? plan->few_tb : 1);
-  plan->few_split = (int)(grp < 1 ? 1 : grp < cu ? grp : cu);
-  const size_t part = (size_t)plan->few_split * N * 4;
+  const int64_t grp = (V + 31) / 32;
+  plan->few_split = few_runs(plan->few_tb, grp);
+  // with the active tokens counted on the device: any smaller number of token blocks, in at most
+  // kFewRounds rounds or one run each
+  const int64_t wgs = active ? (plan->few_tb > kFewRounds * kFwdRound ? plan->few_tb : kFewRounds * kFwdRound)
+                             : (int64_t)plan->few_tb * plan->few_split;
+  const int64_t cap = (int64_t)plan->few_tb * few_runs_max(1, grp);
+  plan->few_wgs = (int)(wgs < cap ? wgs : cap);
+  const size_t part = (size_t)plan->few_wgs * 32 * plan->few_NB * 4;
   const size_t tb = two ? 2 : 4;
   const int sk = two ? SliceK<bf16_t>::value : SliceK<float>::value;
-  size_t off = 0;
   plan->few_m = off;
   off += align256(part);
   plan->few_l = off;
@@ -1015,20 +1021,16 @@ void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, FwdPlan*
   if (off > plan->ws_bytes) plan->ws_bytes = off;
 }
 
-// Whether the call takes the few-token forward: an fp32 W's line, and 32-bit offsets that reach 128
-// rows of W and E.
+// Whether the call takes the few-token forward: planned so, and 32-bit offsets reach 128 rows of W and E.
 bool few_fits(const FwdPlan& plan, const FwdParams& p, int dtype) {
   const int64_t esz = dtype == kF32 ? 4 : 2, wsz = p.w_f32 ? 4 : esz, lim = (int64_t)1 << 31;
-  return plan.few && (!p.w_f32 || p.N <= kFewTokensF32W) && p.ldw * wsz * 128 < lim && p.lde * esz * 128 < lim;
+  return plan.few && p.ldw * wsz * 128 < lim && p.lde * esz * 128 < lim;
 }
 
-// With weight set (a weighted loss), a finite O element or LSE of a zero-weight token is written as 0.
-template <class T>
-hipError_t fwd_few_typed(int dtype, const FwdPlan& plan, const FwdParams& p, const float* weight, char* ws, float* O,
-                         float* lse, float* m_out, float* l_out, hipStream_t stream) {
-  T* const hp = reinterpret_cast<T*>(ws + plan.few_hp);
+// Workspace pointers and sizes of the few-token kernel's parameters.
+FwdFewParams few_params(const FwdPlan& plan, const FwdParams& p, char* ws) {
   FwdFewParams q{};
-  q.hp = hp;
+  q.hp = ws + plan.few_hp;
   q.hS = plan.hS;
   q.W = p.W;
   q.ldw = p.ldw;
@@ -1042,31 +1044,49 @@ hipError_t fwd_few_typed(int dtype, const FwdPlan& plan, const FwdParams& p, con
   q.NB = plan.few_NB;
   q.n_tb = plan.few_tb;
   q.n_split = plan.few_split;
+  q.n_wg = plan.few_tb * plan.few_split;
   q.part_m = reinterpret_cast<float*>(ws + plan.few_m);
   q.part_l = reinterpret_cast<float*>(ws + plan.few_l);
   q.part_acc = reinterpret_cast<float*>(ws + plan.few_acc);
+  return q;
+}
+
+// One pass of the few-token kernel over E's columns from d0 on (E's rows as 16-byte chunks: the
+// caller's, or an aligned copy).
+template <class T>
+hipError_t few_pass(int dtype, const FwdPlan& plan, const FwdParams& p, int d0, FwdFewParams q, char* ws,
+                    hipStream_t stream) {
+  const T* E = static_cast<const T*>(p.E) + d0;
+  q.D = p.D - d0 < plan.DS ? p.D - d0 : plan.DS;
+  q.E = E;
+  q.lde = p.lde;
+  if (p.V > 0 && q.D > 0 && !(rows_vec16(E, p.lde) && q.D % (16 / (int)sizeof(T)) == 0)) {
+    T* const Ep = reinterpret_cast<T*>(ws + plan.few_E);
+    const int64_t n = (int64_t)p.V * (plan.few_DP / 8);
+    timing_begin(kKindPack, stream);
+    pack_vocab_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(
+        E, p.lde, nullptr, p.V, q.D, p.V, plan.few_DP, rows_vec16(E, p.lde), Ep, nullptr);
+    timing_end(kKindPack, stream);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    q.E = Ep;
+    q.lde = plan.few_DP;
+    q.D = plan.few_DP;
+  }
+  return fwd_few_launch(dtype, q, stream);
+}
+
+// With weight set (a weighted loss), a finite O element or LSE of a zero-weight token is written as 0.
+template <class T>
+hipError_t fwd_few_typed(int dtype, const FwdPlan& plan, const FwdParams& p, const float* weight, char* ws, float* O,
+                         float* lse, float* m_out, float* l_out, hipStream_t stream) {
+  const FwdFewParams q = few_params(plan, p, ws);
   timing_begin(kKindPack, stream);
-  hipError_t e = pack_src<T>(p.h, p.h_f32, p.ldh, p.N, p.K, plan.hS, plan.N_pad, hp, stream);
+  hipError_t e = pack_src<T>(p.h, p.h_f32, p.ldh, p.N, p.K, plan.hS, plan.N_pad, reinterpret_cast<T*>(ws + plan.few_hp),
+                             stream);
   timing_end(kKindPack, stream);
   for (int d0 = 0; e == hipSuccess && d0 < (p.D > 0 ? p.D : 1); d0 += plan.DS) {
-    const T* E = static_cast<const T*>(p.E) + d0;
-    q.D = p.D - d0 < plan.DS ? p.D - d0 : plan.DS;
-    q.E = E;
-    q.lde = p.lde;
-    if (p.V > 0 && q.D > 0 && !(rows_vec16(E, p.lde) && q.D % (16 / (int)sizeof(T)) == 0)) {
-      // E's rows as 16-byte chunks, zero past D
-      T* const Ep = reinterpret_cast<T*>(ws + plan.few_E);
-      const int64_t n = (int64_t)p.V * (plan.few_DP / 8);
-      timing_begin(kKindPack, stream);
-      pack_vocab_kernel<T><<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(
-          E, p.lde, nullptr, p.V, q.D, p.V, plan.few_DP, rows_vec16(E, p.lde), Ep, nullptr);
-      timing_end(kKindPack, stream);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-      q.E = Ep;
-      q.lde = plan.few_DP;
-      q.D = plan.few_DP;
-    }
-    if ((e = fwd_few_launch(dtype, q, stream)) != hipSuccess) return e;
+    if ((e = few_pass<T>(dtype, plan, p, d0, q, ws, stream)) != hipSuccess) return e;
     const int D = p.D - d0 < plan.DS ? p.D - d0 : plan.DS;
     e = launch_combine(q.part_m, q.part_l, q.part_acc, q.n_split, p.N, D, (int64_t)plan.few_DP * p.N, p.N, 1,
                        O ? O + d0 : nullptr, p.D, lse, m_out, l_out, weight, stream);
@@ -1157,6 +1177,18 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
   // 2 x n_tb x n_split workgroups' n_tb x BM positions each (active_grid)
   const int64_t NR = active ? 2 * (int64_t)plan->n_tb * BM : N;
   size_t off = 0;
+  plan->off_flag = plan->off_idx = plan->off_inv = plan->off_nact = 0;
+  if (active) {
+    plan->off_flag = off;
+    off += align256((size_t)N * 4);
+    plan->off_idx = off;
+    off += align256((size_t)N * 4);
+    plan->off_inv = off;
+    off += align256((size_t)N * 4);
+    plan->off_nact = off;  // [0] count, [1..2] parameter flags
+    off += 256;
+  }
+  const size_t base = off;  // the general and the few-token forward's buffers, one or the other, follow
   plan->off_m = off;
   off += align256((size_t)parts * NR * 4);
   plan->off_l = off;
@@ -1173,19 +1205,8 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
   off += align256((size_t)plan->N_pad * plan->hS * (tbytes == 4 ? SliceK<float>::value : SliceK<bf16_t>::value) * tbytes);
   plan->off_Wp = off;
   off += align256((size_t)plan->V_pad * plan->hS * (tbytes == 4 ? SliceK<float>::value : SliceK<bf16_t>::value) * tbytes);
-  plan->off_flag = plan->off_idx = plan->off_inv = plan->off_nact = 0;
-  if (active) {
-    plan->off_flag = off;
-    off += align256((size_t)N * 4);
-    plan->off_idx = off;
-    off += align256((size_t)N * 4);
-    plan->off_inv = off;
-    off += align256((size_t)N * 4);
-    plan->off_nact = off;  // [0] count, [1..2] parameter flags
-    off += 256;
-  }
   plan->ws_bytes = off;
-  few_plan(dtype, N, V, Dw, active, plan);
+  few_plan(dtype, N, V, Dw, active, base, plan);
   return true;
 }
 
@@ -1245,14 +1266,56 @@ hipError_t fwd_launch(int dtype, const FwdPlan& plan, FwdParams p, char* ws, flo
 
 namespace {
 
+// Whether W (rows of 16-byte chunks, K a multiple of 8) holds an infinity or a NaN in the compute
+// dtype, for a forward that does not pack it: bad[0] = 1 (as fwd_param_scan_kernel).
+template <class Src, class T>
+__global__ __launch_bounds__(256) void fwd_w_scan_kernel(const Src* __restrict__ W, int64_t ldw, int V, int K,
+                                                         int* __restrict__ bad) {
+  constexpr int CE = 16 / (int)sizeof(T);
+  bool nf = false;
+  for (int v = blockIdx.x; v < V; v += gridDim.x)
+    for (int c = threadIdx.x; c < K / CE; c += 256)
+      nf |= chunk_nonfinite<T>(load_chunk<Src, T>(W + (int64_t)v * ldw + (int64_t)c * CE));
+  if (__syncthreads_or(nf) && threadIdx.x == 0) bad[0] = 1;
+}
+
+// The few-token forward's token blocks and vocabulary runs (few_runs) for the count, into n_act[3],
+// n_act[4]; one wave, a candidate per lane.
+__global__ __launch_bounds__(64) void fwd_few_grid_kernel(int* __restrict__ n_act, int BM, int grp) {
+  const int n = n_act[0], tb = (n + BM - 1) / BM;
+  int64_t best = INT64_MAX;
+  int pick = 1;
+  if (tb > 0)
+    for (int s = 1 + (int)threadIdx.x; s <= few_runs_max(tb, grp); s += 64) {
+      const int64_t t = few_span(tb, grp, s);
+      if (t < best) {
+        best = t;
+        pick = s;
+      }
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const int64_t t = __shfl_xor(best, o);
+    const int q = __shfl_xor(pick, o);
+    if (t < best || (t == best && q < pick)) {
+      best = t;
+      pick = q;
+    }
+  }
+  if (threadIdx.x == 0) {
+    n_act[3] = tb;
+    n_act[4] = pick;
+  }
+}
+
 // Everything of the active-token forward before its passes: the parameter flags (bad[0..1], set
-// while W is packed and by the E / bias scan), the per-token flags and their compaction into
+// while W is packed, or with few by a scan of it, and by the E / bias scan), the per-token flags and their compaction into
 // positions (idx, inv, n_act[0]), the device-side token blocks and splits (n_act[3..4]), and the
 // active tokens' h rows packed in position order.  n_act points at the count block:
 // [0] count, [1..2] parameter flags, [3..4] token blocks and splits.
 template <class T>
 hipError_t active_setup(const FwdPlan& plan, const FwdParams& p, const float* weight, int* flag, int* idx, int* inv,
-                        int* n_act, int* bad, hipStream_t stream) {
+                        int* n_act, int* bad, bool few, T* hp, hipStream_t stream) {
   timing_begin(kKindPack, stream);
   const bool scale_bad = !std::isfinite(p.scale);
   fwd_flags_init_kernel<<<1, 64, 0, stream>>>(bad, scale_bad ? 1 : 0, (p.bias || p.V == 0) ? 1 : 0);
@@ -1261,7 +1324,18 @@ hipError_t active_setup(const FwdPlan& plan, const FwdParams& p, const float* we
   PackExtra wx;
   wx.nonfinite = bad;
   T* const Wp = const_cast<T*>(static_cast<const T*>(p.Wp));
-  if (e == hipSuccess) e = pack_src<T>(p.W, p.w_f32, p.ldw, p.V, p.K, plan.hS, plan.V_pad, Wp, stream, nullptr, wx);
+  if (few) {
+    if (e == hipSuccess && p.V > 0 && p.K > 0) {
+      const unsigned blocks = p.V < 2048 ? p.V : 2048;
+      if (sizeof(T) == 2 && p.w_f32)
+        fwd_w_scan_kernel<float, T><<<blocks, 256, 0, stream>>>(static_cast<const float*>(p.W), p.ldw, p.V, p.K, bad);
+      else
+        fwd_w_scan_kernel<T, T><<<blocks, 256, 0, stream>>>(static_cast<const T*>(p.W), p.ldw, p.V, p.K, bad);
+      e = hipGetLastError();
+    }
+  } else if (e == hipSuccess) {
+    e = pack_src<T>(p.W, p.w_f32, p.ldw, p.V, p.K, plan.hS, plan.V_pad, Wp, stream, nullptr, wx);
+  }
   const int64_t work = (int64_t)p.V * (p.D > 0 ? p.D : 1);
   if (e == hipSuccess && work > 0 && (p.D > 0 || p.bias)) {
     const int blocks = (int)((work + 255) / 256 < 2048 ? (work + 255) / 256 : 2048);
@@ -1280,14 +1354,16 @@ hipError_t active_setup(const FwdPlan& plan, const FwdParams& p, const float* we
   }
   if (e == hipSuccess) e = compact_tokens(flag, p.N, idx, inv, n_act, stream);
   if (e == hipSuccess) {
-    fwd_active_grid_kernel<<<1, 64, 0, stream>>>(n_act, plan.BM, plan.n_tb, plan.n_split, plan.n_vt);
+    if (few)
+      fwd_few_grid_kernel<<<1, 64, 0, stream>>>(n_act, 32 * plan.few_NB, (p.V + 31) / 32);
+    else
+      fwd_active_grid_kernel<<<1, 64, 0, stream>>>(n_act, plan.BM, plan.n_tb, plan.n_split, plan.n_vt);
     e = hipGetLastError();
   }
   // h rows of the active tokens in position order, zeros past them
   PackExtra hx;
   hx.rows = idx;
   hx.n_rows = n_act;
-  T* const hp = const_cast<T*>(static_cast<const T*>(p.hp));
   if (e == hipSuccess) e = pack_src<T>(p.h, p.h_f32, p.ldh, p.N, p.K, plan.hS, plan.N_pad, hp, stream, nullptr, hx);
   timing_end(kKindPack, stream);
   return e;
@@ -1299,7 +1375,9 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
                              float* lse, hipStream_t stream) {
   if (p.N == 0) return hipSuccess;
   if (!plan.active || dtype == kFP8) return hipErrorInvalidValue;
-  if (few_fits(plan, p, dtype)) return fwd_few(dtype, plan, p, weight, ws, O, lse, nullptr, nullptr, stream);
+  const bool few = few_fits(plan, p, dtype);
+  if (few && p.N <= (dtype == kF32 ? kFewTokensActiveF32 : kFewTokensActive))
+    return fwd_few(dtype, plan, p, weight, ws, O, lse, nullptr, nullptr, stream);
   p.n_tb = plan.n_tb;
   p.n_split = plan.n_split;
   p.n_vt = plan.n_vt;
@@ -1316,11 +1394,15 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
   int* inv = reinterpret_cast<int*>(ws + plan.off_inv);
   int* n_act = reinterpret_cast<int*>(ws + plan.off_nact);
   p.n_act = n_act;
+  FwdFewParams fq = few_params(plan, p, ws);
+  fq.n_act = n_act;
+  fq.n_wg = plan.few_wgs;
+  void* const hp = few ? ws + plan.few_hp : ws + plan.off_hp;
   hipError_t e;
   switch (dtype) {
-    case kBF16: e = active_setup<bf16_t>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, stream); break;
-    case kF16: e = active_setup<f16_t>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, stream); break;
-    case kF32: e = active_setup<float>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, stream); break;
+    case kBF16: e = active_setup<bf16_t>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, few, static_cast<bf16_t*>(hp), stream); break;
+    case kF16: e = active_setup<f16_t>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, few, static_cast<f16_t*>(hp), stream); break;
+    case kF32: e = active_setup<float>(plan, p, weight, flag, idx, inv, n_act, n_act + 1, few, static_cast<float*>(hp), stream); break;
     default: return hipErrorInvalidValue;
   }
   if (e != hipSuccess) return e;
@@ -1330,19 +1412,26 @@ hipError_t fwd_launch_active(int dtype, const FwdPlan& plan, FwdParams p, const 
     FwdParams q = p;
     q.E = static_cast<const char*>(p.E) + d0 * esz;
     q.D = D - d0 < plan.DS ? D - d0 : plan.DS;
-    switch (dtype) {
+    switch (few ? 4 + dtype : dtype) {
       case kBF16: e = pack_et<bf16_t>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<bf16_t>(plan, q, stream); break;
       case kF16: e = pack_et<f16_t>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<f16_t>(plan, q, stream); break;
-      default: e = pack_et<float>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<float>(plan, q, stream); break;
+      case kF32: e = pack_et<float>(q, plan, stream); if (e == hipSuccess) e = dispatch_dp<float>(plan, q, stream); break;
+      case 4 + kBF16: e = few_pass<bf16_t>(dtype, plan, p, d0, fq, ws, stream); break;
+      case 4 + kF16: e = few_pass<f16_t>(dtype, plan, p, d0, fq, ws, stream); break;
+      default: e = few_pass<float>(dtype, plan, p, d0, fq, ws, stream); break;
     }
     if (e != hipSuccess) return e;
+    const float* const cm = few ? fq.part_m : p.part_m;
+    const float* const cl = few ? fq.part_l : p.part_l;
+    const float* const ca = few ? fq.part_acc : p.part_acc;
+    const int cBM = few ? 32 * plan.few_NB : plan.BM, cWV = few ? 1 : plan.WV, cDP = few ? plan.few_DP : plan.DP;
     timing_begin(kKindFwdCombine, stream);
     auto go = [&](auto g, auto dt) {
       constexpr int G = decltype(g)::value, DT = decltype(dt)::value;
       fwd_combine_active_kernel<G, DT><<<combine_blocks<G, DT>(p.N, q.D), G * MergeWidth<G>::value, 0, stream>>>(
-          p.part_m, p.part_l, p.part_acc, inv, n_act, plan.BM, plan.WV, p.N, q.D, plan.DP, O + d0, D, lse);
+          cm, cl, ca, inv, n_act, cBM, cWV, p.N, q.D, cDP, O + d0, D, lse);
     };
-    dispatch_combine((int64_t)p.N * q.D, plan.n_part, go);
+    dispatch_combine((int64_t)p.N * q.D, few ? plan.few_split : plan.n_part, go);
     timing_end(kKindFwdCombine, stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }

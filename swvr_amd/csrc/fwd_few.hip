@@ -1,9 +1,13 @@
-// Forward for few tokens: O = softmax(s * h W^T + b) E and LSE when the call is
-// bound by reading W once, not by its matrix work.
+// Forward that streams W as it is stored: O = softmax(s * h W^T + b) E and LSE of
+// few tokens, bound by reading W once and not by matrix work, and of any number
+// in fp32.
 //
 // The general forward (fwd.hip) packs W into its tiles' LDS image first, which
 // pays where many token blocks read it but moves W's bytes three times, and its
-// tiles of 128 or 256 tokens are mostly padding here.  This kernel streams W's
+// tiles of 128 or 256 tokens are mostly padding here.  In fp32, where a matrix
+// instruction takes 16 times as long and the operand traffic hardly counts, this
+// kernel's 128 x 128 tile of 8 waves is the faster one at any size: 8192 tokens on
+// V = 32000, K = 2560, D = 64 13.3 -> 10.7 ms (129 TF/s).  This kernel streams W's
 // rows as the caller stores them (rounding an fp32 W to the compute dtype at
 // the operand read), E's rows likewise, and the bias:
 //   * a workgroup owns a run of vocabulary rows (whole 32-row groups; one
@@ -104,7 +108,7 @@ struct FewCfg {
   typedef FewETile<T, DP, NT> TE;
   static constexpr int FIT = (kLdsBytes - TE::BYTES) / SB;
   static constexpr int NS = FIT < 8 ? FIT : 8;
-  static_assert(NS >= 3 && (NS - 2) * L < 64, "ring depth");
+  static_assert(NS >= 2 && (NS - 2) * L < 64, "ring depth");
   static constexpr int LDS = NS * SB + TE::BYTES;
   // the merge of the waves' partials reuses the LDS: 4 x [DP][32] floats, then 4 x [32 NB] of three
   static_assert(kFewWV * (DP * 32 + 3 * 32 * NB) * 4 <= LDS, "merge fits");
@@ -138,11 +142,18 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
 
   const int lane = lane_id(), w = wave_id(), wv = w % kFewWV, wt = w / kFewWV;
   // an XCD works through a contiguous range of runs, a run's token blocks side by side: they share W in its L2
-  const int t = xcd_swizzle(blockIdx.x, p.n_tb * p.n_split);
-  const int split = t / p.n_tb, n0 = (t % p.n_tb) * 32 * NB;
+  int n_tb = p.n_tb, n_split = p.n_split, ntok = p.N;  // ntok: token rows of a partial
+  if (p.n_act) {
+    n_tb = p.n_act[3];
+    n_split = p.n_act[4];
+    if ((int)blockIdx.x >= n_tb * n_split) return;
+    ntok = n_tb * 32 * NB;
+  }
+  const int t = xcd_swizzle(blockIdx.x, n_tb * n_split);
+  const int split = t / n_tb, n0 = (t % n_tb) * 32 * NB;
   const int n_grp = (p.V + 31) / 32;
-  const int v_begin = (int)((int64_t)split * n_grp / p.n_split) * 32;
-  const int v_end = min(p.V, (int)((int64_t)(split + 1) * n_grp / p.n_split) * 32);
+  const int v_begin = (int)((int64_t)split * n_grp / n_split) * 32;
+  const int v_end = min(p.V, (int)((int64_t)(split + 1) * n_grp / n_split) * 32);
   const int n_tiles = v_end > v_begin ? (v_end - v_begin + kFewBV - 1) / kFewBV : 0;
   const int nk = max(1, (p.K + BK - 1) / BK);  // K = 0: one all-zero slice (bias-only scores)
   const int total = n_tiles * nk;
@@ -339,14 +350,14 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       for (int e = threadIdx.x; e < DP * 32; e += NT) {
         const int n = n0 + (bt * FT + ft) * 32 + (e & 31);
         const float a = ((sA[e] + sA[DP * 32 + e]) + sA[2 * DP * 32 + e]) + sA[3 * DP * 32 + e];
-        if (n < p.N) p.part_acc[((int64_t)split * DP + (e >> 5)) * p.N + n] = a;
+        if (n < ntok) p.part_acc[((int64_t)split * DP + (e >> 5)) * ntok + n] = a;
       }
-      if (w == 0 && lane < 32 && n0 + c < p.N) {
+      if (w == 0 && lane < 32 && n0 + c < ntok) {
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < kFewWV; ++j) sum += sL[j * 32 * NB + c] * fast_exp(sS[j * 32 * NB + c] - shift);
-        p.part_m[(int64_t)split * p.N + n0 + c] = M;
-        p.part_l[(int64_t)split * p.N + n0 + c] = sum;
+        p.part_m[(int64_t)split * ntok + n0 + c] = M;
+        p.part_l[(int64_t)split * ntok + n0 + c] = sum;
       }
       __syncthreads();
     }
@@ -356,7 +367,7 @@ template <class T, class WS, int DP, int FT, int WT>
 hipError_t launch(const FwdFewParams& p, hipStream_t stream) {
   if (p.n_tb * 32 * FT * WT < p.N) return hipErrorInvalidValue;
   timing_begin(kKindFwdTile, stream);
-  fwd_few_kernel<T, WS, DP, FT, WT><<<p.n_tb * p.n_split, FewCfg<T, WS, DP, FT, WT>::NT, 0, stream>>>(p);
+  fwd_few_kernel<T, WS, DP, FT, WT><<<p.n_wg, FewCfg<T, WS, DP, FT, WT>::NT, 0, stream>>>(p);
   timing_end(kKindFwdTile, stream);
   return hipGetLastError();
 }
@@ -367,7 +378,7 @@ hipError_t dispatch_nb(const FwdFewParams& p, hipStream_t stream) {
     case 1: return launch<T, WS, DP, 1, 1>(p, stream);
     case 2: return launch<T, WS, DP, 1, 2>(p, stream);
     case 4:
-      if constexpr (sizeof(T) == 2 && DP <= 128) return launch<T, WS, DP, 2, 2>(p, stream);
+      if constexpr (DP <= 128) return launch<T, WS, DP, 2, 2>(p, stream);
       return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
@@ -376,6 +387,9 @@ hipError_t dispatch_nb(const FwdFewParams& p, hipStream_t stream) {
 template <class T, class WS>
 hipError_t dispatch_dp(const FwdFewParams& p, hipStream_t stream) {
   switch (p.DP) {
+    case 32:
+      if constexpr (sizeof(T) == 4) return dispatch_nb<T, WS, 32>(p, stream);
+      return hipErrorInvalidValue;
     case 64: return dispatch_nb<T, WS, 64>(p, stream);
     case 128: return dispatch_nb<T, WS, 128>(p, stream);
     case 256:

@@ -107,7 +107,7 @@ struct FwdPlan {
   int rem_DP, rem_BM, rem_tb, rem_split, rem_part;
   // few tokens (fwd_few.hip): tile, split and workspace of that path; few = false: not taken
   bool few;
-  int few_DP, few_NB, few_tb, few_split;
+  int few_DP, few_NB, few_tb, few_split, few_wgs;  // few_wgs: workgroups the partials hold
   size_t few_m, few_l, few_acc, few_hp, few_E;
 };
 
@@ -141,12 +141,34 @@ struct FwdFewParams {
   const float* bias;   // [V] or null
   float scale;
   int N, K, V, D;
-  int DP, NB;          // padded D (64, 128, 256), 32-token blocks per workgroup (1, 2, 4)
+  int DP, NB;          // padded D (32 fp32 only, 64, 128, 256), 32-token blocks per workgroup (1, 2, 4)
   int n_tb, n_split;   // token blocks, vocabulary runs
-  float* part_m;       // [n_split][N]
+  int n_wg;            // workgroups to launch (n_tb x n_split, or with n_act as many as may be needed)
+  // active tokens only: hp holds their rows in position order, [3] / [4] of this device block the token
+  // blocks and runs (few_runs); null: every token at its own row
+  const int* n_act;
+  float* part_m;       // [n_split][N] (with n_act, rows of [3] x 32 NB positions)
   float* part_l;
   float* part_acc;     // [n_split][DP][N]
 };
+
+// Vocabulary runs of the few-token forward for n_tb token blocks over grp 32-row groups, when one
+// workgroup runs per CU: the count that ends soonest, each workgroup taking its longest run and about
+// one group's time more for its ring fill and partial stores, over at most kFewRounds rounds of the CUs.
+constexpr int kFewRounds = 4;
+__host__ __device__ inline int64_t few_span(int64_t n_tb, int64_t grp, int64_t s) {
+  return (n_tb * s + kFwdRound - 1) / kFwdRound * ((grp + s - 1) / s + 1);
+}
+__host__ __device__ inline int few_runs_max(int64_t n_tb, int64_t grp) {
+  const int64_t m = kFewRounds * kFwdRound / (n_tb > 0 ? n_tb : 1), c = m < grp ? m : grp;
+  return c < 1 ? 1 : (int)c;
+}
+inline int few_runs(int64_t n_tb, int64_t grp) {
+  int best = 1;
+  for (int s = 2; s <= few_runs_max(n_tb, grp); ++s)
+    if (few_span(n_tb, grp, s) < few_span(n_tb, grp, best)) best = s;
+  return best;
+}
 hipError_t fwd_few_launch(int dtype, const FwdFewParams& p, hipStream_t stream);
 
 // Order-preserving compaction of flagged tokens (flag[n] != 0): idx[q] = token

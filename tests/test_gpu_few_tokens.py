@@ -85,7 +85,7 @@ def test_compaction_of_active_tokens_over_workgroups(N):
 @pytest.mark.parametrize("N,K,V,D", [
     (1, 72, 20011, 64), (31, 8, 97, 8), (32, 512, 9001, 200), (33, 40, 31, 128), (64, 1032, 5000, 33),
     (65, 264, 16385, 64), (128, 100, 4097, 72), (129, 96, 8193, 256), (255, 2048, 600, 300), (256, 64, 1, 16),
-    (769, 64, 900, 64), (1024, 136, 2000, 130),
+    (768, 64, 900, 64), (769, 136, 2000, 130),
 ])
 def test_few_token_forward(dtype, N, K, V, D):
     amp = dtype == "autocast"
@@ -168,3 +168,27 @@ def test_last_pass_of_wide_embeddings_on_a_narrower_kernel(dtype, N, K, V, D):
     for sl in (slice(0, D // 256 * 256), slice(D // 256 * 256, D)):
         assert sl.start == sl.stop or rel_err(O[:, sl], torch.softmax(S, -1) @ E.double()[:, sl]) <= bar
     assert rel_err(lse, torch.logsumexp(S, -1)) <= bar
+
+
+# the few-token kernel over the active tokens' positions (fp32 at any size, 2-byte types between 512 and
+# 768 tokens): the device picks blocks and runs for the count, from none to all, at the edges of a block
+@pytest.mark.parametrize("dtype,N", [(torch.float32, 2500), (torch.float32, 129), (torch.bfloat16, 700)])
+@pytest.mark.parametrize("count", [0, 1, 127, 129, 10**6])
+@pytest.mark.parametrize("V,D", [(3001, 20), (31, 140)])
+def test_active_positions_on_the_few_token_kernel(dtype, N, count, V, D):
+    from swvr_amd import _ops
+    h, W, E, b = make(N, 72, V, D, dtype, requires_grad=False)
+    w = torch.zeros(N, device="cuda")
+    w[torch.randperm(N, generator=torch.Generator().manual_seed(1))[:count].cuda()] = 0.5
+    O, lse = _ops._forward_active(h, W, E, b, w, 1.0, 8192, dtype)
+    on = w != 0
+    assert (O[~on] == 0).all() and (lse[~on] == 0).all()
+    if count:
+        S = h[on].double() @ W.double().T + b.double()
+        bar = 1e-5 if dtype == torch.float32 else 1e-2
+        assert rel_err(O[on], torch.softmax(S, -1) @ E.double()) <= bar
+        assert rel_err(lse[on], torch.logsumexp(S, -1)) <= bar
+    W2 = W.clone()
+    W2[V - 1, 71] = float("nan")   # a parameter's NaN keeps every token computed, as the reference's loss needs
+    O, lse = _ops._forward_active(h, W2, E, b, w, 1.0, 8192, dtype)
+    assert O.isnan().all() and lse.isnan().all()
