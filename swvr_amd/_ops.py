@@ -15,6 +15,8 @@ from typing import List, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -305,8 +307,112 @@ def _autograd_backward_active(ctx, gO, glse):
 _fwd_active_op.register_autograd(_autograd_backward_active, setup_context=_setup_context_active)
 
 
+# ---------------------------------------------------------------- eager calls
+def eager(*tensors):
+    """Whether a call on these tensors (None allowed) may go to the library without the custom ops: plain
+    GPU tensors, and nothing looking at the ops themselves (compilation, tracing, functorch transforms,
+    forward-mode AD, dispatch or function modes).  The custom ops' own Python layers take about 40 us of
+    host time per op and direction, of the 480 that a training step of 512 tokens in fp32 (N = 512,
+    K = 256, V = 4096) took when its kernels take 160; without them, and with the loss in the readout's
+    node (``readout_mse_eager``), it takes 270."""
+    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0):
+        return False
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.device.type == "cuda")
+               for t in tensors)
+
+
+def _needs_grad(*tensors):
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def _save(ctx, tensors, args):
+    ctx.save_for_backward(*tensors)
+    ctx.args = args
+    ctx.set_materialize_grads(False)
+
+
+def _readout_grads(ctx, gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt):
+    """The four gradients, None where not needed (as ``_autograd_backward``)."""
+    needs = [bool(n) for n in ctx.needs_input_grad[:4]]
+    needs[3] = needs[3] and bias is not None
+    gO = gO if gO is not None else torch.zeros_like(O)
+    glse = glse if glse is not None else torch.zeros_like(lse)
+    return _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, *needs)
+
+
+class _Readout(torch.autograd.Function):
+    """swvr::chunked_fwd / chunked_bwd, or with a weight swvr::chunked_fwd_active, as one node."""
+
+    @staticmethod
+    def forward(ctx, h, W, E, bias, weight, logit_scale, chunk, cdt):
+        if weight is None:
+            O, lse = _forward(h, W, E, bias, logit_scale, chunk, cdt)
+        else:
+            O, lse = _forward_active(h, W, E, bias, weight, logit_scale, chunk, cdt)
+        _save(ctx, (h, W, E, bias, O, lse), (logit_scale, chunk, cdt))
+        return O, lse
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gO, glse):
+        grads = _readout_grads(ctx, gO, glse, *ctx.saved_tensors, *ctx.args)
+        return (*grads, None, None, None, None)
+
+
+class _ReadoutMse(torch.autograd.Function):
+    """The readout and swvr::mse_loss on it as one node, returning the loss."""
+
+    @staticmethod
+    def forward(ctx, h, W, E, bias, target, weight, active, z, reduction, logit_scale, chunk, cdt):
+        if active:
+            O, lse = _forward_active(h, W, E, bias, weight, logit_scale, chunk, cdt)
+        else:
+            O, lse = _forward(h, W, E, bias, logit_scale, chunk, cdt)
+        out, scale, gO, glse = _mse_loss(O, lse, target, weight, z, reduction, True)
+        _save(ctx, (h, W, E, bias, O, lse, scale, gO, glse), (reduction, logit_scale, chunk, cdt))
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        if g is None:
+            return (None,) * 12
+        h, W, E, bias, O, lse, scale, gO, glse = ctx.saved_tensors
+        reduction, *args = ctx.args
+        gO, glse = _mse_scaled(g, scale, gO, glse, reduction)
+        grads = _readout_grads(ctx, gO, glse, h, W, E, bias, O, lse, *args)
+        return (*grads, None, None, None, None, None, None, None, None)
+
+
+def readout_mse_eager(h2, W, E, bias, target2, weight, active, z, reduction, logit_scale, chunk, cdt):
+    """The loss of a call that ``eager`` lets through: h2 [N, K], target2 [N, D], weight [N] or None;
+    active: the forward over the tokens of non-zero weight.  [N] for "none", else a scalar."""
+    red = REDUCTIONS[reduction]
+    if _needs_grad(h2, W, E, bias):
+        return _ReadoutMse.apply(h2, W, E, bias, target2, weight, active, float(z), red, float(logit_scale),
+                                 int(chunk), cdt)
+    if active:
+        O, lse = _forward_active(h2, W, E, bias, weight, float(logit_scale), int(chunk), cdt)
+    else:
+        O, lse = _forward(h2, W, E, bias, float(logit_scale), int(chunk), cdt)
+    return _mse_loss(O, lse, target2, weight, float(z), red, False)[0]
+
+
+def _readout_eager(h2, W, E, bias, weight, logit_scale, chunk, cdt):
+    args = (float(logit_scale), int(chunk), cdt)
+    if _needs_grad(h2, W, E, bias):
+        return _Readout.apply(h2, W, E, bias, weight, *args)
+    if weight is None:
+        return _forward(h2, W, E, bias, *args)
+    return _forward_active(h2, W, E, bias, weight, *args)
+
+
 def softmax_readout_op(h2, W, E, bias, logit_scale, chunk, cdt):
     """``h2`` is ``[N, K]``; returns ``(O [N, D], LSE [N])`` in fp32 (swvr/chunked.py:208-212)."""
+    if eager(h2, W, E, bias):
+        return _readout_eager(h2, W, E, bias, None, logit_scale, chunk, cdt)
     if h2.device.type not in ("cuda", "cpu"):  # meta / fake tracing: no autocast state
         return _fwd_op(h2, W, E, bias, float(logit_scale), int(chunk), cdt, True)
     with torch.autocast(h2.device.type, enabled=False):
@@ -316,6 +422,8 @@ def softmax_readout_op(h2, W, E, bias, logit_scale, chunk, cdt):
 def softmax_readout_active_op(h2, W, E, bias, weight, logit_scale, chunk, cdt):
     """``softmax_readout_op`` for a weighted loss: tokens with ``weight == 0`` get O rows and lse
     of 0 instead of their readout (``swvr_fwd_active``); ``weight`` is [N], no gradient."""
+    if eager(h2, W, E, bias, weight):
+        return _readout_eager(h2, W, E, bias, weight, logit_scale, chunk, cdt)
     if h2.device.type not in ("cuda", "cpu"):
         return _fwd_active_op(h2, W, E, bias, weight, float(logit_scale), int(chunk), cdt)
     with torch.autocast(h2.device.type, enabled=False):
@@ -382,12 +490,16 @@ def _mse_setup_context(ctx, inputs, output):
     ctx.reduction = reduction
 
 
-def _mse_autograd_backward(ctx, g, _g_scale, _g_gO, _g_glse):
-    scale, gO, glse = ctx.saved_tensors
-    if ctx.reduction == 0:
-        return gO * g[:, None], glse * g, None, None, None, None, None
+def _mse_scaled(g, scale, gO, glse, reduction):
+    """The loss's derivatives times the reduction's factor and the incoming gradient."""
+    if reduction == 0:
+        return gO * g[:, None], glse * g
     s = g * scale
-    return gO * s, glse * s, None, None, None, None, None
+    return gO * s, glse * s
+
+
+def _mse_autograd_backward(ctx, g, _g_scale, _g_gO, _g_glse):
+    return (*_mse_scaled(g, *ctx.saved_tensors, ctx.reduction), None, None, None, None, None)
 
 
 _mse_op.register_autograd(_mse_autograd_backward, setup_context=_mse_setup_context)

@@ -10,7 +10,8 @@ import os
 import torch
 from torch import nn
 
-from ._ops import DEFAULT_CHUNK, REDUCTIONS, mse_loss_op, softmax_readout_active_op, softmax_readout_op
+from ._ops import (DEFAULT_CHUNK, REDUCTIONS, eager, mse_loss_op, readout_mse_eager, softmax_readout_active_op,
+                   softmax_readout_op)
 
 
 def default_chunk_size():
@@ -55,12 +56,19 @@ def softmax_readout(h, W, E, bias=None, *, logit_scale=1.0, chunk_size=None):
     """
     _check(h, W, E, bias)
     lead = h.shape[:-1]
-    h2 = h.reshape(-1, h.shape[-1])
+    h2 = _rows(h)
     chunk = int(chunk_size) if chunk_size else default_chunk_size()
     if chunk <= 0:
         raise ValueError(f"chunk_size must be positive, got {chunk}")
     O, lse = softmax_readout_op(h2, W, E, bias, logit_scale, chunk, _compute_dtype(h, W))
+    if h2 is h:
+        return O, lse
     return O.view(*lead, E.shape[1]), lse.view(lead)
+
+
+def _rows(h):
+    """``h`` as [tokens, K]: itself when it is (no view node for autograd to walk)."""
+    return h if h.dim() == 2 and h.shape[1] > 0 else h.reshape(-1, h.shape[-1])
 
 
 def softmax_readout_mse(h, W, E, target, bias=None, *, weight=None, reduction="mean",
@@ -73,7 +81,16 @@ def softmax_readout_mse(h, W, E, target, bias=None, *, weight=None, reduction="m
     weighted sum over the sum of the weights, or over the token count without weights),
     "sum", or "none" (the per-token values).
     """
-    if _skips_zero_weight(h, W, weight, reduction):
+    skips = _skips_zero_weight(h, W, weight, reduction)
+    if _one_call(h, W, E, target, bias, weight, reduction):
+        _check(h, W, E, bias)
+        chunk = int(chunk_size) if chunk_size else default_chunk_size()
+        if chunk <= 0:
+            raise ValueError(f"chunk_size must be positive, got {chunk}")
+        out = readout_mse_eager(_rows(h), W, E, bias, _rows(target), weight.reshape(-1) if weight is not None else None,
+                                skips, z_loss_weight, reduction, logit_scale, chunk, _compute_dtype(h, W))
+        return out.view(h.shape[:-1]) if reduction == "none" else out
+    if skips:
         # The loss is weight x (a finite term) per token, so zero-weight tokens need no readout:
         # the library computes the others only and gives these O rows and lse of 0, for which
         # the term is finite again (swvr_fwd_active lists the rows it still computes to keep
@@ -89,6 +106,18 @@ def softmax_readout_mse(h, W, E, target, bias=None, *, weight=None, reduction="m
     else:
         O, lse = softmax_readout(h, W, E, bias, logit_scale=logit_scale, chunk_size=chunk_size)
     return _mse_loss(O, lse, target, weight, reduction, z_loss_weight)
+
+
+def _one_call(h, W, E, target, bias, weight, reduction):
+    """Whether the readout and the loss on it go to the library in one step (``readout_mse_eager``):
+    an eager call on tensors of the right shapes whose loss the library's kernels compute
+    (``_fusable_loss`` on the O and lse that the readout would give)."""
+    if not all(isinstance(x, torch.Tensor) for x in (h, W, E, target)) or not eager(h, W, E, target, bias, weight):
+        return False
+    if W.dim() != 2 or E.dim() != 2 or h.dim() < 1 or reduction not in REDUCTIONS:
+        return False
+    return (_compute_dtype(h, W) in (torch.bfloat16, torch.float16, torch.float32)
+            and _loss_inputs_fusable(h.shape[:-1], E.shape[1], h.device, target, weight))
 
 
 def _skips_zero_weight(h, W, weight, reduction):
@@ -136,12 +165,18 @@ def _fusable_loss(O, lse, target, weight, reduction):
         return False
     if O.dtype != torch.float32 or lse.dtype != torch.float32:  # the loss kernels read fp32 (fp64 readouts: composite)
         return False
-    if not isinstance(target, torch.Tensor) or target.shape != O.shape or target.device != O.device:
+    return _loss_inputs_fusable(lse.shape, O.shape[-1], O.device, target, weight)
+
+
+def _loss_inputs_fusable(lead, D, device, target, weight):
+    if D < 1 or lead.numel() == 0:
+        return False
+    if not isinstance(target, torch.Tensor) or target.shape != (*lead, D) or target.device != device:
         return False
     if target.requires_grad or target.is_complex():
         return False
     if weight is not None:
-        if not isinstance(weight, torch.Tensor) or weight.shape != lse.shape or weight.device != O.device:
+        if not isinstance(weight, torch.Tensor) or weight.shape != lead or weight.device != device:
             return False
         if weight.requires_grad or weight.is_complex():
             return False
