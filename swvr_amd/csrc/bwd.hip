@@ -137,8 +137,8 @@ __global__ __launch_bounds__(1024) void bwd_compact_kernel(const int* __restrict
 }
 
 // The token-side operands of the scores kernel over positions: gO rounded to
-// the compute dtype (swvr/chunked.py:115) as [N_pad][DP] (zero padded), the
-// same values transposed per token block as [N_pad / BM][DP][BM] with the
+// the compute dtype (swvr/chunked.py:115) as [N_pad][DP] (zero padded), with gOt
+// set (the scores kernels that read it) the same values transposed per token block as [N_pad / BM][DP][BM] with the
 // positions of a block in pe_row order (the A operand of dE^T = gO^T P), and
 // [lse | delta] as 2 x N_pad floats (lse = +inf on padding: P = 0 there).
 template <class T>
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void bwd_pack_kernel(const float* __restrict__
   const int q = (int)(e / DP), d = (int)(e % DP);
   const int n = q < na ? idx[q] : -1;
   gOp[e] = (n >= 0 && d < D) ? from_float<T>(gO[(int64_t)n * D + d]) : (T)0.f;
-  {
+  if (gOt) {
     const int64_t blk = e / ((int64_t)DP * BM);
     const int rem = (int)(e - blk * DP * BM);
     const int dt = rem / BM;
@@ -305,11 +305,17 @@ struct ScoresTile {
   static constexpr int WT = wide && DP == 128 ? 2 : 1;
   static constexpr int WV = 4;
   static constexpr int NT = 64 * WT * WV;
-  // LDS: the K-slice ring plus E [BV][DP], gO [BM][DP], gO^T [DP][BM], bias
+  // fp32 reads the gO^T operand of dE from the gO tile, element by element (its matrix work takes 16
+  // times as long); the 2-byte types from a gO^T tile of its own.  Without that tile the ring at
+  // D = 128 is 4 slots deep instead of 2 (4096 tokens, K = 1024, V = 16384: 2.20 -> 1.59 ms, 108 TF/s)
+  // and D = 32 and 64 fit two workgroups on a CU (2048 tokens, K = 1024, V = 20000, D = 16: 0.89 -> 0.76).
+  static constexpr bool GT = wide;
+  // LDS: the K-slice ring plus E [BV][DP], gO [BM][DP], gO^T [DP][BM] (GT), bias
   // and LSE / delta; the ring is as deep as the 160 KB allow (at most 4).
-  static constexpr int SIDE = (BV + 2 * BM) * DP * (int)sizeof(T) + BV * 4 + 2 * BM * 4;
+  static constexpr int SIDE = (BV + (GT ? 2 : 1) * BM) * DP * (int)sizeof(T) + BV * 4 + 2 * BM * 4;
   static constexpr int SB = (BM + BV) * 64;
-  static constexpr int NS = SIDE + 4 * SB <= 160 * 1024 ? 4 : SIDE + 3 * SB <= 160 * 1024 ? 3 : 2;
+  static constexpr int LDS = !wide && SIDE + 2 * SB <= 80 * 1024 ? 80 * 1024 : 160 * 1024;  // two workgroups, or one
+  static constexpr int NS = SIDE + 4 * SB <= LDS ? 4 : SIDE + 3 * SB <= LDS ? 3 : 2;
 };
 
 // One workgroup: BV vocabulary rows of the chunk x one group of token
@@ -339,11 +345,13 @@ __global__ __launch_bounds__((ScoresTile<T, DP>::NT)) void bwd_scores_kernel(Sco
   constexpr int DB = DP / 32, DK = DP / 16;
 
   constexpr int NS = C::NS;
-  __shared__ __attribute__((aligned(1024))) char smem[NS * SB + TE::BYTES + TG::BYTES + TGT::BYTES + BV * 4 + 2 * BM * 4];
+  constexpr bool GT = C::GT;
+  constexpr int GTB = GT ? TGT::BYTES : 0;
+  __shared__ __attribute__((aligned(1024))) char smem[NS * SB + TE::BYTES + TG::BYTES + GTB + BV * 4 + 2 * BM * 4];
   char* const sE = smem + NS * SB;
   char* const sG = sE + TE::BYTES;
   char* const sGt = sG + TG::BYTES;
-  float* const sBias = reinterpret_cast<float*>(sGt + TGT::BYTES);
+  float* const sBias = reinterpret_cast<float*>(sGt + GTB);
   float* const sLse = sBias + BV;
   float* const sDelta = sLse + BM;
 
@@ -362,7 +370,7 @@ __global__ __launch_bounds__((ScoresTile<T, DP>::NT)) void bwd_scores_kernel(Sco
   // E and bias of the vocabulary tile: once per workgroup, ahead of the stages
   const uint32_t lds0 = lds_addr(smem);
   const uint32_t ldsE = lds0 + NS * SB, ldsG = ldsE + TE::BYTES, ldsGt = ldsG + TG::BYTES;
-  const uint32_t ldsB = ldsGt + TGT::BYTES;
+  const uint32_t ldsB = ldsGt + GTB;
   const uint32_t ldsL = ldsB + BV * 4;
   {
     TE te;
@@ -417,9 +425,11 @@ __global__ __launch_bounds__((ScoresTile<T, DP>::NT)) void bwd_scores_kernel(Sco
       TG tg;
       tg.setup(static_cast<const T*>(p.gOp) + (int64_t)n0 * DP, DP, BM, DP);
       tg.issue(ldsG, 0);
-      TGT tgt;
-      tgt.setup(static_cast<const T*>(p.gOt) + (int64_t)n0 * DP, BM, DP, BM);
-      tgt.issue(ldsGt, 0);
+      if constexpr (GT) {
+        TGT tgt;
+        tgt.setup(static_cast<const T*>(p.gOt) + (int64_t)n0 * DP, BM, DP, BM);
+        tgt.issue(ldsGt, 0);
+      }
       const int c = threadIdx.x;  // BM/4 chunks of LSE, then BM/4 of delta
       if (c < BM / 2) {
         const uint32_t off = c < BM / 4 ? (uint32_t)(n0 + 4 * c) * 4 : (uint32_t)(p.N_pad + n0 + 4 * (c - BM / 4)) * 4;
@@ -500,10 +510,10 @@ __global__ __launch_bounds__((ScoresTile<T, DP>::NT)) void bwd_scores_kernel(Sco
               if constexpr (sizeof(T) == 2) {
                 av = *reinterpret_cast<const V8*>(sGte + TGT::elem(d, p0));
               } else {
-                const float4 lo = *reinterpret_cast<const float4*>(sGte + TGT::elem(d, p0));
-                const float4 hi = *reinterpret_cast<const float4*>(sGte + TGT::elem(d, p0 + 4));
-                av[0] = lo.x; av[1] = lo.y; av[2] = lo.z; av[3] = lo.w;
-                av[4] = hi.x; av[5] = hi.y; av[6] = hi.z; av[7] = hi.w;
+#pragma unroll
+                for (int tt = 0; tt < 8; ++tt)
+                  av[tt] = *reinterpret_cast<const float*>(
+                      sGe + TG::elem(tr0 + 16 * c + 8 * (tt >> 2) + 4 * (lane >> 5) + (tt & 3), d));
               }
               mfma_k16(deacc[db][fv], av, bv);
             }
@@ -1670,6 +1680,7 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
   T* hqc = reinterpret_cast<T*>(ws + plan.off_hqc);
   float* multp = f8 ? reinterpret_cast<float*>(ws + plan.off_mult) : nullptr;
   const bool need_stage = p.gh || p.gW;
+  const bool reads_gOt = plan.kind == kScoresRing || f8;  // see ScoresTile::GT; the wide kernel forms no dE
   const int dh_split = p.gW ? plan.dh_split_w : plan.dh_split_h;
   const bool gemm_de = pstage && p.gE;  // dE^T = gO^T P as tiles of the gradient GEMM launch
   // every chunk has a gradient GEMM launch: the W packing of the scores kernel rides on them
@@ -1682,8 +1693,8 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
     if ((e = compact_tokens(flag, p.N, idx, inv, n_act, stream)) != hipSuccess) return e;
     const int64_t n = (int64_t)plan.N_pad * plan.DP;
     bwd_pack_kernel<T><<<(int)((n + 255) / 256), 256, 0, stream>>>(p.gO, p.lse, delta, idx, n_act, p.D,
-                                                                   (int)plan.N_pad, plan.DP, plan.BM, gOp, gOt,
-                                                                   lsed);
+                                                                   (int)plan.N_pad, plan.DP, plan.BM, gOp,
+                                                                   reads_gOt ? gOt : nullptr, lsed);
     timing_end(kKindBwdDelta, stream);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const int64_t nv = (int64_t)plan.V_pad * (plan.DP / 8);
