@@ -147,7 +147,9 @@ int swvr_combine(int64_t S, int64_t N, int64_t D, const float* m, const float* l
 
 /* Workspace bytes swvr_bwd needs.  `chunk` is the vocabulary staging chunk
  * (the reference's chunk_size, swvr/chunked.py:120): the backward stages
- * dS for `chunk` vocabulary rows at a time, so this is O(N * chunk). */
+ * dS for `chunk` vocabulary rows at a time, so this is O(N * chunk).  Fewer
+ * than 4096 tokens stage several chunks of 8192 rows or more together, up to
+ * the memory 4096 tokens would take (swvr_bwd_tiling reports the rows). */
 size_t swvr_bwd_workspace_size(int dtype, int64_t N, int64_t K, int64_t V, int64_t D,
                                int64_t chunk, int need_gh);
 
@@ -202,7 +204,7 @@ int swvr_bwd_f64(int64_t N, int64_t K, int64_t V, int64_t D, const double* h, in
  * scores kernel; [1] BV, its vocabulary tile; [2] G, the token groups a
  * vocabulary tile's token blocks are split over (one workgroup per group, so a
  * workgroup walks ceil(active token blocks / G) blocks); [3] C, the vocabulary
- * rows per chunk; [4] the number of chunks; [5] DP, the padded embedding
+ * rows staged together (a chunk, or several with few tokens); [4] how many such; [5] DP, the padded embedding
  * width; [6] the scores kernel: 1 the narrow-embedding kernel (side tiles
  * carried by its K ring), 2 the wide-embedding kernel (gO and E streamed as
  * D-slices; dE formed by the gradient GEMM launch), 0 the general one.

@@ -167,10 +167,10 @@ __global__ __launch_bounds__(256) void bwd_pack_kernel(const float* __restrict__
   }
 }
 
-// h rows of the active tokens in position order, [N_pad][K] (zeros past
-// n_act), 16 bytes of T per thread; h may be fp32 for a 2-byte T (rounded here).
-template <class Src, class T>
-__global__ __launch_bounds__(256) void bwd_gather_rows_kernel(const Src* __restrict__ h, int64_t ldh,
+// Rows of h (the e4m3 backward's: plain, or e4m3 bytes as pairs) of the active tokens in position
+// order, [N_pad][K] (zeros past n_act), 16 bytes per thread.
+template <class T>
+__global__ __launch_bounds__(256) void bwd_gather_rows_kernel(const T* __restrict__ h, int64_t ldh,
                                                               const int* __restrict__ idx,
                                                               const int* __restrict__ n_act, int N_pad, int K,
                                                               T* __restrict__ hc) {
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void bwd_gather_rows_kernel(const Src* __restr
   const int q = (int)(e / cpr), c = (int)(e % cpr);
   const int n = q < n_act[0] ? idx[q] : -1;
   uint4 v = make_uint4(0, 0, 0, 0);
-  if (n >= 0) v = load_chunk<Src, T>(h + (int64_t)n * ldh + (int64_t)c * CE);
+  if (n >= 0) v = *reinterpret_cast<const uint4*>(h + (int64_t)n * ldh + (int64_t)c * CE);
   *reinterpret_cast<uint4*>(hc + (int64_t)q * K + (int64_t)c * CE) = v;
 }
 
@@ -1704,22 +1704,17 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
                                                                            plan.DP, rows_vec16(E, p.lde), Ep, biasp,
                                                                            p.h_scale, p.w_scale, p.scale, multp);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (p.K > 0) {
-      const int64_t nh = plan.N_pad * (p.K / (16 / (int)sizeof(T)));
-      const unsigned gb = (unsigned)((nh + 255) / 256);
-      if (sizeof(T) == 2 && p.h_f32)
-        bwd_gather_rows_kernel<float, T><<<gb, 256, 0, stream>>>(static_cast<const float*>(p.h), p.ldh, idx,
-                                                                  n_act, (int)plan.N_pad, p.K, hc);
-      else
-        bwd_gather_rows_kernel<T, T><<<gb, 256, 0, stream>>>(static_cast<const T*>(p.h), p.ldh, idx, n_act,
-                                                              (int)plan.N_pad, p.K, hc);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
     if (f8) {
+      if (p.K > 0) {
+        const int64_t nh = plan.N_pad * (p.K / (16 / (int)sizeof(T)));
+        bwd_gather_rows_kernel<T><<<(unsigned)((nh + 255) / 256), 256, 0, stream>>>(
+            static_cast<const T*>(p.h), p.ldh, idx, n_act, (int)plan.N_pad, p.K, hc);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+      }
       // the scores kernel reads the e4m3 operands; the gradient GEMMs keep h over positions and W
       const int k2 = p.K8 / 2;
       const int64_t nq = plan.N_pad * (k2 / (16 / (int)sizeof(T)));
-      bwd_gather_rows_kernel<T, T><<<(unsigned)((nq + 255) / 256), 256, 0, stream>>>(
+      bwd_gather_rows_kernel<T><<<(unsigned)((nq + 255) / 256), 256, 0, stream>>>(
           static_cast<const T*>(p.hq), p.ldhq / 2, idx, n_act, (int)plan.N_pad, k2, hqc);
       if ((e = hipGetLastError()) != hipSuccess) return e;
       if ((e = launch_pack_rows<T>(hqc, k2, (int)plan.N_pad, k2, plan.hS8, plan.N_pad, hp, stream)) != hipSuccess)
@@ -1728,7 +1723,12 @@ hipError_t bwd_run(const BwdPlan& plan, const BwdParams& p, hipStream_t stream) 
           hipSuccess)
         return e;
     } else {
-      if ((e = launch_pack_rows<T>(hc, p.K, (int)plan.N_pad, p.K, plan.hS, plan.N_pad, hp, stream)) != hipSuccess)
+      // h over positions, packed for the scores kernel and plain for the dW product, in one pass over
+      // h (a gather of its own and a packing of its result read it twice more)
+      PackExtra hx;
+      hx.rows = idx;
+      hx.n_rows = n_act;
+      if ((e = pack_src<T>(p.h, p.h_f32, p.ldh, p.N, p.K, plan.hS, plan.N_pad, hp, stream, hc, hx)) != hipSuccess)
         return e;
       // Wp holds one chunk's packed rows: the first chunk's are packed here; chunk c + 1's by
       // chunk c's gradient GEMM launch (gemm_pack_w) after chunk c's scores kernel has read its
@@ -1913,6 +1913,22 @@ hipError_t compact_tokens(const int* flag, int N, int* idx, int* inv, int* n_act
   return hipGetLastError();
 }
 
+// Chunks of the vocabulary that a backward of few tokens stages together.  Each chunk costs a scores
+// and a GEMM launch, which few token blocks leave mostly idle (500 tokens, K = 1024: 64 scores workgroups
+// and 256 short GEMM tiles per 8192 rows), and one more read and write of every dh accumulator.  So
+// fewer than 4096 tokens stage as many rows as 4096 tokens' memory at the given chunk holds, the packed
+// rows of W staying within 256 MB.  A chunk below the default of 8192 rows asks for less memory and is
+// kept as it is.  Steps, one chunk at a time -> together: 500 tokens, K = 1024, V = 32000 (all 4 chunks)
+// 418 -> 317 us; 2048 tokens, K = 1024, V = 151936, gradient of h alone (pairs) 2.60 -> 2.32 ms; 1332 in
+// fp32, K = 768, V = 30001 (pairs) 2.65 -> 2.49.
+constexpr int64_t kChunkDefault = 8192, kChunkTokens = 4096, kChunkPackBytes = (int64_t)256 << 20;
+int64_t chunks_together(int64_t N_pad, int64_t K, int64_t chunk, int64_t tb) {
+  if (chunk < kChunkDefault || N_pad >= kChunkTokens || chunk > ((int64_t)1 << 22)) return 1;
+  const int64_t by_tokens = kChunkTokens / N_pad, by_pack = kChunkPackBytes / (chunk * (K > 0 ? K : 1) * tb);
+  const int64_t n = by_tokens < by_pack ? by_tokens : by_pack;
+  return n > 1 ? n : 1;
+}
+
 bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chunk, bool need_gh, BwdPlan* plan,
               bool w_f32, int64_t K8) {
   const bool f8 = K8 > 0;
@@ -1965,7 +1981,8 @@ bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chu
   plan->n_tb = (int)((N + BM - 1) / BM);
   plan->N_pad = ((N + 255) / 256) * 256;
   if (plan->N_pad == 0) plan->N_pad = 256;
-  int64_t c = chunk < V ? chunk : V;
+  int64_t c = chunk * chunks_together(plan->N_pad, K, chunk, two ? 2 : 4);
+  if (c > V) c = V;
   // at most 2^22 rows per chunk: tile-relative offsets into [DP or rows][C] buffers stay 32-bit
   if (c > ((int64_t)1 << 22)) c = (int64_t)1 << 22;
   if (c < 1) c = 1;

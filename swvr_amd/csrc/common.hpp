@@ -1001,7 +1001,8 @@ __device__ __forceinline__ bool chunk_nonfinite(uint4 v) {
 // The source may be fp32 for a 2-byte T (rounded here); with rowmajor set,
 // the rows are also written as a plain [N][K] copy in T.  With rows set, packed
 // row q is source row rows[q] for q < n_rows[0] and zero past it (a gather of
-// selected tokens in position order).  With nonfinite set, a workgroup that
+// selected tokens in position order), and so is row q of the plain copy, up to
+// the padded row count.  With nonfinite set, a workgroup that
 // packs an infinity or a NaN stores 1 there (every such store writes the same
 // value, so the word ends as 1 whatever their order).
 // One 32-row x 8-slice tile `grp_s` (32-row group grp_s / SG, slices from (grp_s % SG) * 8)
@@ -1033,9 +1034,10 @@ __device__ __forceinline__ bool pack_rows_tile(int grp_s, int t, uint4* tile, co
     uint4 v = make_uint4(0, 0, 0, 0);
     if (kc < ns * CPR && n >= 0 && k < K) {
       v = load_chunk<Src, T>(src + n * ld + k);
-      if (rowmajor) *reinterpret_cast<uint4*>(rowmajor + n * K + k) = v;
+      if (rowmajor && !rows) *reinterpret_cast<uint4*>(rowmajor + n * K + k) = v;
       bad |= chunk_nonfinite<T>(v);
     }
+    if (rowmajor && rows && kc < ns * CPR && k < K) *reinterpret_cast<uint4*>(rowmajor + q * K + k) = v;
     tile[row * RSTRIDE + kc] = v;
   }
   __syncthreads();

@@ -192,3 +192,12 @@ def test_active_positions_on_the_few_token_kernel(dtype, N, count, V, D):
     W2[V - 1, 71] = float("nan")   # a parameter's NaN keeps every token computed, as the reference's loss needs
     O, lse = _ops._forward_active(h, W2, E, b, w, 1.0, 8192, dtype)
     assert O.isnan().all() and lse.isnan().all()
+
+
+# several chunks staged together, and a second such group that is not whole
+@pytest.mark.parametrize("dtype,N,K,V,D", [(torch.bfloat16, 200, 64, 140001, 24), (torch.bfloat16, 1030, 72, 40000, 100),
+                                           (torch.float32, 520, 64, 66000, 16)])
+def test_chunks_staged_together(dtype, N, K, V, D):
+    inputs = make(N, K, V, D, dtype, w_scale=1.0)
+    bars = (1e-2, 2e-2) if dtype == torch.bfloat16 else (1e-5, 1e-5)
+    check(inputs, lambda *a: swvr.softmax_readout(*a, chunk_size=8192), (N,), D, *bars)
