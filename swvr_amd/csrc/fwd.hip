@@ -693,7 +693,9 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ pm, con
 }
 
 // Thread rows G of a merge (DT = 1 with 32, else 4).
-int combine_rows(int64_t elements, int n_part) { return n_part < 64 ? 1 : elements <= 65536 ? 32 : 4; }
+int combine_rows(int64_t elements, int n_part) {
+  return elements <= 65536 && n_part >= 16 ? 32 : n_part < 64 ? 1 : 4;
+}
 
 template <int G, int DT>
 __global__ __launch_bounds__(G * MergeWidth<G>::value) void fwd_combine_kernel(
@@ -951,7 +953,7 @@ namespace {
 // of ring fill and partial stores; a single round ends with its longest, several even out half of that.
 // 2500 tokens on V = 50021, K = 768, D = 256 (20 token blocks): 52 splits are 1040 workgroups, a fifth
 // round for 16 of them, and the pass took 436 us; 25 make 2 whole rounds, 356 us.
-int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int64_t K, int DP, int BM) {
+int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int s_min, int64_t K, int DP, int BM) {
   const double tile = ((double)K + DP) / 32 * 0.3 * (BM / 128.0), over = 5.0;
   auto span = [&](int64_t s) {
     const int64_t rounds = (n_tb * s + kFwdRound - 1) / kFwdRound;
@@ -959,9 +961,9 @@ int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int64_t K, int DP, i
     return rounds * (avg * tile + over) + rest * tile * (rounds > 1 ? 0.5 : 1.0);
   };
   double best = 0.97 * span(n_split);
-  const int64_t cap = n_vt / 2 > 1 ? n_vt / 2 : 1, hi = 4 * (int64_t)kFwdRound / n_tb;
+  const int64_t cap = n_vt / 2 > 1 ? n_vt / 2 : 1, hi = 6 * (int64_t)kFwdRound / n_tb;
   int pick = n_split;
-  for (int64_t s = 1; s <= hi && s <= cap; ++s)
+  for (int64_t s = s_min; s <= hi && s <= cap; ++s)
     if (span(s) < best) {
       best = span(s);
       pick = (int)s;
@@ -1152,7 +1154,9 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
     const int max_split = plan->n_vt / 2 > 1 ? plan->n_vt / 2 : 1;
     if (n_split > max_split) n_split = max_split;
     if (n_split < 1) n_split = 1;
-    if (!active && tbytes == 2 && dtype != kFP8) n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, K, DP, BM);
+    // (the e4m3 forward's P is relative to the running maximum, so it keeps at least the rule's splits)
+    if (!active && tbytes == 2)
+      n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, dtype == kFP8 ? n_split : 1, K, DP, BM);
   }
   plan->n_split = n_split;
   plan->n_part = WV * n_split;
