@@ -52,6 +52,21 @@ def test_merge_of_partials(dtype, N, K, V, D):
     assert O.isnan().all() and (lse == float("-inf")).all()
 
 
+# the same merge where its 32 runs hold no, one or two partials each: a workgroup per 32 vocabulary rows,
+# so V / 32 partials, and a merge of that many shards
+@pytest.mark.parametrize("parts", [15, 16, 17, 31, 32, 33, 63, 64, 65])
+def test_merge_of_few_partials(parts):
+    from swvr_amd import vocab_shard as vs
+    N, K, V, D = 7, 64, 32 * parts - 5, 40
+    h, W, E, b = (x.detach() for x in make(N, K, V, D, torch.float32))
+    b[32 * (parts - 2):] = float("-inf")   # the last two partials hold no score
+    S = h.double() @ W.double().T + b.double()
+    want_O, want_lse = torch.softmax(S, -1) @ E.double(), torch.logsumexp(S, -1)
+    shards = [vs.softmax_readout_partial(h, W[v:v + 32], E[v:v + 32], b[v:v + 32]) for v in range(0, V, 32)]
+    for O, lse in (swvr.softmax_readout(h, W, E, b), vs.combine_partials(*(torch.stack(x) for x in zip(*shards)))):
+        assert rel_err(O, want_O) <= 1e-5 and rel_err(lse, want_lse) <= 1e-5
+
+
 @pytest.mark.parametrize("N", [1, 1023, 1024, 1025, 4097, 300001])
 def test_compaction_of_active_tokens_over_workgroups(N):
     """Weights of 0 drop tokens; the others keep their own rows: sizes at the edges of a workgroup's

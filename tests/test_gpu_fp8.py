@@ -45,6 +45,17 @@ def test_fp8_forward_matches_fp64_on_the_dequantised_operands(N, K, V, D, bias):
     assert eo <= 1e-2 and el <= 1e-5
 
 
+# sizes whose vocabulary splits are balanced over the CUs: 86 -> 106 of 235 tiles (some runs of two tiles,
+# some of three), 61 -> 75 of 196, and 114 -> 137 of 274 (two each)
+@pytest.mark.parametrize("N,K,V,D", [(1500, 512, 60001, 33), (2100, 256, 50001, 128), (1100, 48, 70001, 100)])
+def test_fp8_forward_with_balanced_splits(N, K, V, D):
+    h, W, E, b = make(N, K, V, D)
+    O, lse = fp8.softmax_readout_fp8(h, W, E, b)
+    S = fp8.dequantize(*fp8.quantize_tensor(h)).double() @ fp8.dequantize(*fp8.quantize_rows(W)).double().T + b.double()
+    assert rel_err(O, torch.softmax(S, -1) @ E.double()) <= 1e-2
+    assert rel_err(lse, torch.logsumexp(S, -1)) <= 1e-5
+
+
 @pytest.mark.parametrize("K", [512, 2560])
 def test_fp8_forward_stays_within_e4m3_rounding_of_the_unquantised_readout(K):
     N, V, D = 512, 8192, 64
