@@ -787,15 +787,38 @@ hipError_t launch_combine(const float* m, const float* l, const float* acc, int 
   return hipGetLastError();
 }
 
-// The active-token forward's token blocks and vocabulary splits (active_grid)
-// from the count, into n_act[3], n_act[4]: once per call, for every kernel.
+// The active-token forward's token blocks and vocabulary splits from the count, into n_act[3],
+// n_act[4]: once per call, so every kernel uses the same values and the host needs no copy of them.
+// The launch has room for twice the all-token tiling's workgroups, of which the first n_tb x n_split
+// work; the split is the one fwd_span ends soonest with (the smaller on a tie).  One wave, a candidate
+// per lane.
 __global__ __launch_bounds__(64) void fwd_active_grid_kernel(int* __restrict__ n_act, int BM, int n_tb_max,
-                                                             int n_split0, int n_vt) {
+                                                             int n_split0, int n_vt, FwdCost cost) {
+  int tb = (n_act[0] + BM - 1) / BM, pick = 1;
+  if (tb > n_tb_max) tb = n_tb_max;
+  double best = 1e300;
+  if (tb > 0) {
+    const int hi = active_splits_max(tb, n_tb_max, n_split0, n_vt);
+    for (int s = 1 + (int)threadIdx.x; s <= hi; s += 64) {
+      const double t = fwd_span(tb, n_vt, s, cost);
+      if (t < best) {
+        best = t;
+        pick = s;
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const double t = __shfl_xor(best, o);
+    const int q = __shfl_xor(pick, o);
+    if (t < best || (t == best && q < pick)) {
+      best = t;
+      pick = q;
+    }
+  }
   if (threadIdx.x == 0) {
-    int tb, sp;
-    active_grid(n_act[0], BM, n_tb_max, n_split0, n_vt, &tb, &sp);
     n_act[3] = tb;
-    n_act[4] = sp;
+    n_act[4] = pick;
   }
 }
 
@@ -861,7 +884,7 @@ template <class T, int DP, bool F8 = false>
 hipError_t launch_tile(const FwdPlan& plan, const FwdParams& p, hipStream_t stream) {
   typedef FwdCfg<T, DP, F8> C;
   if (plan.BV != C::BV || plan.BM != C::BM) return hipErrorInvalidValue;
-  // the active-token forward may use up to twice the all-token grid (active_grid); the rest exit at once
+  // the active-token forward may use up to twice the all-token grid (active_splits_max); the rest exit at once
   const int blocks = plan.n_tb * plan.n_split * (p.n_act ? 2 : 1);
   timing_begin(kKindFwdTile, stream);
   if constexpr (!F8 && FwdTile<T, DP>::stream_e)
@@ -948,18 +971,11 @@ hipError_t pack(const FwdParams& p, const FwdPlan& plan, hipStream_t stream) {
 namespace {
 
 // Vocabulary splits of a forward whose workgroups hold a CU each, from the rule's n_split: the split
-// that ends soonest when n_tb x s workgroups run 256 at a time, if it is 3% sooner.  A workgroup takes
-// n_vt / s vocabulary tiles on average ((K + DP) / 32 slices of 0.3 us per 128 tokens each) and about 5 us
-// of ring fill and partial stores; a single round ends with its longest, several even out half of that.
+// that fwd_span ends soonest with, if that is 3% sooner.
 // 2500 tokens on V = 50021, K = 768, D = 256 (20 token blocks): 52 splits are 1040 workgroups, a fifth
 // round for 16 of them, and the pass took 436 us; 25 make 2 whole rounds, 356 us.
-int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int s_min, int64_t K, int DP, int BM) {
-  const double tile = ((double)K + DP) / 32 * 0.3 * (BM / 128.0), over = 5.0;
-  auto span = [&](int64_t s) {
-    const int64_t rounds = (n_tb * s + kFwdRound - 1) / kFwdRound;
-    const double avg = (double)n_vt / s, rest = (double)((n_vt + s - 1) / s) - avg;
-    return rounds * (avg * tile + over) + rest * tile * (rounds > 1 ? 0.5 : 1.0);
-  };
+int balanced_split(int64_t n_tb, int64_t n_vt, int n_split, int s_min, FwdCost cost) {
+  auto span = [&](int64_t s) { return fwd_span(n_tb, n_vt, s, cost); };
   double best = 0.97 * span(n_split);
   const int64_t cap = n_vt / 2 > 1 ? n_vt / 2 : 1, hi = 6 * (int64_t)kFwdRound / n_tb;
   int pick = n_split;
@@ -1156,7 +1172,8 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
     if (n_split < 1) n_split = 1;
     // (the e4m3 forward's P is relative to the running maximum, so it keeps at least the rule's splits)
     if (!active && tbytes == 2)
-      n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, dtype == kFP8 ? n_split : 1, K, DP, BM);
+      n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, dtype == kFP8 ? n_split : 1,
+                               fwd_cost(K, DP, BM, WV));
   }
   plan->n_split = n_split;
   plan->n_part = WV * n_split;
@@ -1178,7 +1195,7 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
     }
   }
   // token rows of a partial: N; the active-token forward's partials hold up to
-  // 2 x n_tb x n_split workgroups' n_tb x BM positions each (active_grid)
+  // 2 x n_tb x n_split workgroups' n_tb x BM positions each (active_splits_max)
   const int64_t NR = active ? 2 * (int64_t)plan->n_tb * BM : N;
   size_t off = 0;
   plan->off_flag = plan->off_idx = plan->off_inv = plan->off_nact = 0;
@@ -1361,7 +1378,8 @@ hipError_t active_setup(const FwdPlan& plan, const FwdParams& p, const float* we
     if (few)
       fwd_few_grid_kernel<<<1, 64, 0, stream>>>(n_act, 32 * plan.few_NB, (p.V + 31) / 32);
     else
-      fwd_active_grid_kernel<<<1, 64, 0, stream>>>(n_act, plan.BM, plan.n_tb, plan.n_split, plan.n_vt);
+      fwd_active_grid_kernel<<<1, 64, 0, stream>>>(n_act, plan.BM, plan.n_tb, plan.n_split, plan.n_vt,
+                                                   fwd_cost(p.K, plan.DP, plan.BM, plan.WV));
     e = hipGetLastError();
   }
   // h rows of the active tokens in position order, zeros past them

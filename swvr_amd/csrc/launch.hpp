@@ -53,41 +53,35 @@ struct FwdParams {
   const float* w_scale;  // e4m3 forward: [V] dequantisation scales of W's rows, else null
   // Active-token forward: [0] the count of active tokens, whose rows are packed
   // in position order (hp), [3] / [4] the token blocks and vocabulary splits
-  // (active_grid), all on the device; null: every token, at its own row.
+  // (fwd_active_grid_kernel), all on the device; null: every token, at its own row.
   const int* n_act;
 };
 
-// Token blocks and vocabulary splits of an active-token forward, from the
-// device count of active tokens.  The launch has grid = n_tb_max x n_split0
-// workgroups (the all-token tiling: whole rounds of kFwdRound, one workgroup
-// per CU); with n_act active tokens the first n_tb x n_split of them work.  The
-// split count minimises the forward's duration in the round model, rounds x
-// vocabulary tiles per workgroup ~ ceil(n_tb x s / kFwdRound) / s, over
-// s = n_split0 .. min(n_vt / 2, 2 x grid / n_tb) (the smallest such s on a
-// tie): the partial buffers hold 2 x grid workgroups' partials.  Computed once
-// per call (fwd_active_grid_kernel) into the count's block, so every kernel of
-// the forward uses the same values and the host needs no copy of them.
 constexpr int kFwdRound = 256;
-__host__ __device__ inline void active_grid(int n_act, int BM, int n_tb_max, int n_split0, int n_vt, int* n_tb,
-                                            int* n_split) {
-  int tb = n_act <= 0 ? 0 : (n_act + BM - 1) / BM;
-  if (tb > n_tb_max) tb = n_tb_max;
-  int sp = n_split0;
-  if (tb > 0) {
-    const int cap = n_vt / 2 > 1 ? n_vt / 2 : 1;
-    const int64_t fit = 2 * (int64_t)n_tb_max * n_split0 / tb;
-    const int hi = fit < cap ? (int)fit : cap;
-    int64_t best_r = ((int64_t)tb * sp + kFwdRound - 1) / kFwdRound;
-    for (int s = n_split0 + 1; s <= hi; ++s) {
-      const int64_t r = ((int64_t)tb * s + kFwdRound - 1) / kFwdRound;
-      if (r * sp < best_r * s) {  // r / s < best_r / sp
-        best_r = r;
-        sp = s;
-      }
-    }
-  }
-  *n_tb = tb;
-  *n_split = sp;
+
+// Model of a forward whose n_tb x s workgroups hold a CU each and run 256 at a time, in units of about
+// 1.5 us: a workgroup takes n_vt / s vocabulary tiles on average, `tile` each, and 5 for its ring fill
+// and partial stores; a single round ends with its longest workgroup, several even out half of that; the
+// merge reads every workgroup's partials, `part` each (0.3 us per MB).
+struct FwdCost {
+  double tile, part;
+};
+inline FwdCost fwd_cost(int64_t K, int DP, int BM, int WV) {
+  return {((double)K + DP) / 32 * 0.3 * (BM / 128.0), 0.2e-6 * 4 * WV * BM * DP};
+}
+__host__ __device__ inline double fwd_span(int64_t n_tb, int64_t n_vt, int64_t s, FwdCost c) {
+  const int64_t rounds = (n_tb * s + kFwdRound - 1) / kFwdRound;
+  const double avg = (double)n_vt / s, rest = (double)((n_vt + s - 1) / s) - avg;
+  return rounds * (avg * c.tile + 5.0) + rest * c.tile * (rounds > 1 ? 0.5 : 1.0) + n_tb * s * c.part;
+}
+
+// Vocabulary splits an active-token forward of tb token blocks may take: at least two vocabulary
+// tiles each, and no more workgroups than twice the all-token tiling's n_tb_max x n_split0, which is
+// what the launch and the partial buffers hold.
+__host__ __device__ inline int active_splits_max(int tb, int n_tb_max, int n_split0, int n_vt) {
+  const int cap = n_vt / 2 > 1 ? n_vt / 2 : 1;
+  const int64_t fit = 2 * (int64_t)n_tb_max * n_split0 / (tb > 0 ? tb : 1);
+  return fit < cap ? (int)fit : cap;
 }
 
 struct FwdPlan {
