@@ -148,8 +148,8 @@ int swvr_combine(int64_t S, int64_t N, int64_t D, const float* m, const float* l
 /* Workspace bytes swvr_bwd needs.  `chunk` is the vocabulary staging chunk
  * (the reference's chunk_size, swvr/chunked.py:120): the backward stages
  * dS for `chunk` vocabulary rows at a time, so this is O(N * chunk).  Fewer
- * than 4096 tokens stage several chunks of 8192 rows or more together, up to
- * the memory 4096 tokens would take (swvr_bwd_tiling reports the rows). */
+ * than 8192 tokens stage several chunks of 8192 rows or more together, up to
+ * the memory 8192 tokens would take (swvr_bwd_tiling reports the rows). */
 size_t swvr_bwd_workspace_size(int dtype, int64_t N, int64_t K, int64_t V, int64_t D,
                                int64_t chunk, int need_gh);
 

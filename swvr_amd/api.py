@@ -52,7 +52,7 @@ def softmax_readout(h, W, E, bias=None, *, logit_scale=1.0, chunk_size=None):
     or fp64 when the products run in fp64.  The [tokens, V] scores never exist in memory;
     the backward recomputes them ``chunk_size`` rows of the vocabulary at a time (default
     8192, or ``SWVR_CHUNK``), which bounds its extra memory by O(tokens * chunk_size); fewer
-    than 4096 tokens take several chunks of 8192 or more at a time, within 4096 tokens' memory.
+    than 8192 tokens take several chunks of 8192 or more at a time, within 8192 tokens' memory.
     Autograd reaches every input that requires a gradient.
     """
     _check(h, W, E, bias)

@@ -1916,17 +1916,23 @@ hipError_t compact_tokens(const int* flag, int N, int* idx, int* inv, int* n_act
 // Chunks of the vocabulary that a backward of few tokens stages together.  Each chunk costs a scores
 // and a GEMM launch, which few token blocks leave mostly idle (500 tokens, K = 1024: 64 scores workgroups
 // and 256 short GEMM tiles per 8192 rows), and one more read and write of every dh accumulator.  So
-// fewer than 4096 tokens stage as many rows as 4096 tokens' memory at the given chunk holds, the packed
+// fewer than 8192 tokens stage as many rows as 8192 tokens' memory at the given chunk holds, the packed
 // rows of W staying within 256 MB.  A chunk below the default of 8192 rows asks for less memory and is
-// kept as it is.  Steps, one chunk at a time -> together: 500 tokens, K = 1024, V = 32000 (all 4 chunks)
-// 418 -> 317 us; 2048 tokens, K = 1024, V = 151936, gradient of h alone (pairs) 2.60 -> 2.32 ms; 1332 in
-// fp32, K = 768, V = 30001 (pairs) 2.65 -> 2.49.
-constexpr int64_t kChunkDefault = 8192, kChunkTokens = 4096, kChunkPackBytes = (int64_t)256 << 20;
+// kept as it is.  Powers of two only: 8192 rows are 32 vocabulary tiles, and 3 or 6 such chunks leave a
+// quarter of the CUs without a scores workgroup (1024 tokens, K = 2560, V = 151936: 6 chunks 3.87 ms, 4
+// 3.67).  Steps, one chunk at a time / 4096 tokens' memory / 8192: 500 tokens, K = 1024, V = 32000 (all 4
+// chunks) 418 / 317 / 317 us; 2048 tokens, K = 1024, V = 151936, gradient of h alone 2.60 / 2.26 / 2.15 ms;
+// 1332 in fp32, K = 768, V = 30001 2.65 / 2.39 / 2.29; 1280 tokens, K = 1024, V = 151936 - / 2.16 / 2.03;
+// 4096, K = 1024, V = 128256, gradient of h alone 3.47 / 3.47 / 3.35.  16384 tokens' memory gives up to
+// 3% more at twice the bytes (1280 tokens 1.97 ms, the others within 1%).
+constexpr int64_t kChunkDefault = 8192, kChunkTokens = 8192, kChunkPackBytes = (int64_t)256 << 20;
 int64_t chunks_together(int64_t N_pad, int64_t K, int64_t chunk, int64_t tb) {
   if (chunk < kChunkDefault || N_pad >= kChunkTokens || chunk > ((int64_t)1 << 22)) return 1;
   const int64_t by_tokens = kChunkTokens / N_pad, by_pack = kChunkPackBytes / (chunk * (K > 0 ? K : 1) * tb);
-  const int64_t n = by_tokens < by_pack ? by_tokens : by_pack;
-  return n > 1 ? n : 1;
+  const int64_t most = by_tokens < by_pack ? by_tokens : by_pack;
+  int64_t n = 1;
+  while (2 * n <= most) n *= 2;
+  return n;
 }
 
 bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chunk, bool need_gh, BwdPlan* plan,
