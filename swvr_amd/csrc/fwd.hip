@@ -692,9 +692,12 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ pm, con
   *L_ = L;
 }
 
-// Thread rows G of a merge (DT = 1 with 32, else 4).
+// Thread rows G of a merge (DT = 1 with 32, else 4).  4 also for 16 to 63 partials whose one-row merge
+// would leave CUs without a workgroup (1100 tokens, D = 100, 48 partials: the call 142 -> 135 us; 2500
+// tokens, D = 300, whose last pass merges 44 columns: 572 -> 564; 2000 tokens, D = 200 is past the line).
 int combine_rows(int64_t elements, int n_part) {
-  return elements <= 65536 && n_part >= 16 ? 32 : n_part < 64 ? 1 : 4;
+  if (n_part < 16) return 1;
+  return elements <= 65536 ? 32 : n_part >= 64 || elements <= 4 * 256 * 256 ? 4 : 1;
 }
 
 template <int G, int DT>

@@ -67,6 +67,16 @@ def test_merge_of_few_partials(parts):
         assert rel_err(O, want_O) <= 1e-5 and rel_err(lse, want_lse) <= 1e-5
 
 
+# the merge in 4 runs of 16 to 63 partials, up to 2^18 values (the third and fourth: both sides of that)
+@pytest.mark.parametrize("N,V,D", [(1100, 12001, 100), (769, 6000, 97), (2048, 8001, 128), (2049, 8001, 128)])
+def test_merge_of_some_partials(N, V, D):
+    h, W, E, b = (x.detach() for x in make(N, 64, V, D, torch.float16))
+    b[V // 3:2 * V // 3] = float("-inf")
+    O, lse = swvr.softmax_readout(h, W, E, b)
+    S = h.double() @ W.double().T + b.double()
+    assert rel_err(O, torch.softmax(S, -1) @ E.double()) <= 1e-2 and rel_err(lse, torch.logsumexp(S, -1)) <= 1e-5
+
+
 @pytest.mark.parametrize("N", [1, 1023, 1024, 1025, 4097, 300001])
 def test_compaction_of_active_tokens_over_workgroups(N):
     """Weights of 0 drop tokens; the others keep their own rows: sizes at the edges of a workgroup's
