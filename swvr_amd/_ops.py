@@ -39,9 +39,23 @@ def _kpad(K):
     return (K + 7) // 8 * 8
 
 
+def _plain(x):
+    """``x`` with its values in memory as they are read by pointer: autograd hands out, and callers may
+    pass, views whose sign is still to be flipped (``z.conj().imag``) and zeros without memory, which only
+    the dispatcher resolves; ``.to`` and ``.contiguous()`` return such a one-element view as it is."""
+    x = x.resolve_neg()
+    return x.clone() if x._is_zerotensor() else x
+
+
+def _f32(x):
+    """``x`` as a dense fp32 tensor (or None)."""
+    return None if x is None else _plain(x).to(torch.float32).contiguous()
+
+
 def _matrix(x, cdt, Kp):
     """``x`` [R, K] in the compute dtype with K padded to Kp, unit inner stride,
     16-byte aligned rows (the C ABI's alignment contract)."""
+    x = _plain(x)
     if x.dtype != cdt:
         x = x.to(cdt)
     if x.shape[1] != Kp:
@@ -57,6 +71,7 @@ def _operand(x, cdt, Kp):
     """``(tensor, dtype tag)`` of h or W for the C ABI: an fp32 matrix under a 2-byte compute
     dtype (autocast with fp32 weights) goes as it is, and the kernels round it while packing;
     anything else goes through ``_matrix``."""
+    x = _plain(x)
     if (x.dtype == torch.float32 and cdt in (torch.bfloat16, torch.float16) and x.shape[1] == Kp
             and x.stride(1) == 1 and (x.shape[0] <= 1 or x.stride(0) % 8 == 0) and x.data_ptr() % 16 == 0):
         return x, _lib.F32
@@ -64,6 +79,7 @@ def _operand(x, cdt, Kp):
 
 
 def _embed(E, cdt):
+    E = _plain(E)
     if E.dtype != cdt:
         E = E.to(cdt)
     return E if E.stride(1) == 1 else E.contiguous()
@@ -79,7 +95,7 @@ def _f64(x):
     """``x`` in fp64 with unit stride in its last dimension (or None)."""
     if x is None:
         return None
-    x = x.to(torch.float64)
+    x = _plain(x).to(torch.float64)
     return x if x.dim() < 2 or x.stride(-1) == 1 else x.contiguous()
 
 
@@ -112,8 +128,7 @@ def _backward_f64(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, need_h, n
     gW = torch.empty(V, K, dtype=f64, device=dev) if need_W else None
     gE = torch.empty(V, D, dtype=f64, device=dev) if need_E else None
     gb = torch.empty(V, dtype=f64, device=dev) if need_b else None
-    gOd, glsed = gO.to(f64).contiguous(), glse.to(f64).contiguous()
-    Od, lsed = O.to(f64).contiguous(), lse.to(f64).contiguous()
+    gOd, glsed, Od, lsed = (_plain(x).to(f64).contiguous() for x in (gO, glse, O, lse))
     ws_bytes = lib.swvr_bwd_f64_workspace_size(N, V, D, int(chunk))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
@@ -138,7 +153,7 @@ def _forward(h, W, E, bias, logit_scale, chunk, cdt):
     V, D = E.shape
     Kp = _kpad(K)
     (hc, h_tag), (Wc, w_tag), Ec = _operand(h, cdt, Kp), _operand(W, cdt, Kp), _embed(E, cdt)
-    b = bias.to(torch.float32).contiguous() if bias is not None else None
+    b = _f32(bias)
     O = torch.empty(N, D, dtype=torch.float32, device=h.device)
     lse = torch.empty(N, dtype=torch.float32, device=h.device)
     tag = _lib.DTYPE_TAG[cdt]
@@ -163,8 +178,8 @@ def _forward_active(h, W, E, bias, weight, logit_scale, chunk, cdt):
     V, D = E.shape
     Kp = _kpad(K)
     (hc, h_tag), (Wc, w_tag), Ec = _operand(h, cdt, Kp), _operand(W, cdt, Kp), _embed(E, cdt)
-    b = bias.to(torch.float32).contiguous() if bias is not None else None
-    w = weight.reshape(-1).to(torch.float32).contiguous()
+    b = _f32(bias)
+    w = _f32(weight.reshape(-1))
     O = torch.empty(N, D, dtype=torch.float32, device=h.device)
     lse = torch.empty(N, dtype=torch.float32, device=h.device)
     tag = _lib.DTYPE_TAG[cdt]
@@ -195,16 +210,13 @@ def _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, need_h, 
     V, D = E.shape
     Kp = _kpad(K)
     (hc, h_tag), (Wc, w_tag), Ec = _operand(h, cdt, Kp), _operand(W, cdt, Kp), _embed(E, cdt)
-    b = bias.to(torch.float32).contiguous() if bias is not None else None
+    b = _f32(bias)
     dev = h.device
     gh = _grad_buffer((N, Kp), h.dtype, dev) if need_h else None
     gW = _grad_buffer((V, Kp), W.dtype, dev) if need_W else None
     gE = _grad_buffer((V, D), E.dtype, dev) if need_E else None
     gb = torch.empty(V, dtype=torch.float32, device=dev) if need_b else None
-    gO32 = gO.to(torch.float32).contiguous()
-    glse32 = glse.to(torch.float32).contiguous()
-    O32 = O.to(torch.float32).contiguous()
-    lse32 = lse.to(torch.float32).contiguous()
+    gO32, glse32, O32, lse32 = _f32(gO), _f32(glse), _f32(O), _f32(lse)
     tag = _lib.DTYPE_TAG[cdt]
     ws_bytes = lib.swvr_bwd_workspace_size_mixed(tag, w_tag, N, Kp, V, D, int(chunk), int(need_h))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
@@ -441,12 +453,13 @@ def _mse_loss(O, lse, target, weight, z, reduction, need_grad):
     _require_device(O)
     lib = _lib.load()
     N, D = O.shape
-    O = O.contiguous()
-    lse = lse.contiguous()
-    t = target if target.dtype in _lib.DTYPE_TAG else target.to(torch.float32)
+    O = _plain(O).contiguous()
+    lse = _plain(lse).contiguous()
+    t = _plain(target)
+    t = t if t.dtype in _lib.DTYPE_TAG else t.to(torch.float32)
     if t.stride(1) != 1 or (N > 1 and t.stride(0) < D):
         t = t.contiguous()
-    w = weight.to(torch.float32).contiguous() if weight is not None else None
+    w = _f32(weight)
     dev = O.device
     out = torch.empty((N,) if reduction == 0 else (), dtype=torch.float32, device=dev)
     scale = torch.empty((), dtype=torch.float32, device=dev)

@@ -23,7 +23,7 @@ h and W (the quantisation passes gradients through as the identity).
 import torch
 
 from . import _lib
-from ._ops import _grad_buffer, _kpad, _lead_stride, _matrix, _require_device
+from ._ops import _embed, _f32, _grad_buffer, _kpad, _lead_stride, _matrix, _plain, _require_device
 
 E4M3 = torch.float8_e4m3fn
 E4M3_MAX = 448.0
@@ -33,7 +33,7 @@ def _quantize(x, per_row):
     """``swvr_quantize_e4m3`` of a [R, K] matrix: (e4m3 [R, Kp], fp32 scales), Kp = K padded to 16."""
     _require_device(x)
     lib = _lib.load()
-    x = x.detach()
+    x = _plain(x.detach())
     if x.dtype not in _lib.DTYPE_TAG:
         x = x.to(torch.float32)
     if x.stride(-1) != 1:
@@ -72,9 +72,8 @@ def _fwd(hq, hs, Wq, ws, E, bias, logit_scale):
     lib = _lib.load()
     N, Kq = hq.shape
     V, D = E.shape
-    Eb = E.detach().to(torch.bfloat16)
-    Eb = Eb if Eb.stride(-1) == 1 else Eb.contiguous()
-    b = bias.detach().to(torch.float32).contiguous() if bias is not None else None
+    Eb = _embed(E.detach(), torch.bfloat16)
+    b = _f32(bias.detach()) if bias is not None else None
     O = torch.empty(N, D, dtype=torch.float32, device=hq.device)
     lse = torch.empty(N, dtype=torch.float32, device=hq.device)
     ws_bytes = lib.swvr_fwd_fp8_workspace_size(N, Kq, V, D)
@@ -99,17 +98,15 @@ def _bwd(gO, glse, h, W, E, bias, O, lse, hq, hs, Wq, ws, logit_scale, chunk, ne
     Kp = _kpad(K)
     hb = _matrix(h.detach(), torch.bfloat16, Kp)
     Wb = _matrix(W.detach(), torch.bfloat16, Kp)
-    Eb = E.detach().to(torch.bfloat16)
-    Eb = Eb if Eb.stride(-1) == 1 else Eb.contiguous()
-    b = bias.detach().to(torch.float32).contiguous() if bias is not None else None
+    Eb = _embed(E.detach(), torch.bfloat16)
+    b = _f32(bias.detach()) if bias is not None else None
     need_h, need_W, need_E, need_b = needs
     dev = h.device
     gh = _grad_buffer((N, Kp), h.dtype, dev) if need_h else None
     gW = _grad_buffer((V, Kp), W.dtype, dev) if need_W else None
     gE = _grad_buffer((V, D), E.dtype, dev) if need_E else None
     gb = torch.empty(V, dtype=torch.float32, device=dev) if need_b else None
-    gO32 = gO.to(torch.float32).contiguous()
-    glse32 = glse.to(torch.float32).contiguous()
+    gO32, glse32 = _f32(gO), _f32(glse)
     Kq = hq.shape[1]
     ws_bytes = lib.swvr_bwd_fp8_workspace_size(N, Kp, Kq, V, D, int(chunk), int(need_h))
     work = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
@@ -182,7 +179,7 @@ def softmax_readout_fp8(h, W, E, bias=None, *, logit_scale=1.0, w_q=None, chunk_
         raise ValueError(f"w_q must be quantize_rows(W) of a [{V}, {W.shape[1]}] W on {h.device}")
     # the kernels read dense rows of Kp bytes and fp32 scales
     Wq = Wq.contiguous()
-    ws = ws.to(device=h.device, dtype=torch.float32).contiguous()
+    ws = _f32(ws.to(device=h.device))
     chunk = int(chunk_size) if chunk_size else default_chunk_size()
     if chunk <= 0:
         raise ValueError(f"chunk_size must be positive, got {chunk}")

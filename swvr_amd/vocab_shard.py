@@ -24,7 +24,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._ops import _backward, _embed, _kpad, _lead_stride, _matrix, _require_device
+from ._ops import _backward, _embed, _f32, _kpad, _lead_stride, _matrix, _require_device
 from .api import _check, _compute_dtype, default_chunk_size
 
 
@@ -45,7 +45,7 @@ def softmax_readout_partial(h: torch.Tensor, W: torch.Tensor, E: torch.Tensor, b
     V, D = E.shape
     Kp = _kpad(K)
     hc, Wc, Ec = _matrix(h2, cdt, Kp), _matrix(W, cdt, Kp), _embed(E, cdt)
-    b = bias.to(torch.float32).contiguous() if bias is not None else None
+    b = _f32(bias)
     m = torch.empty(N, dtype=torch.float32, device=h.device)
     l = torch.empty(N, dtype=torch.float32, device=h.device)
     acc = torch.empty(N, D, dtype=torch.float32, device=h.device)
@@ -71,8 +71,7 @@ def combine_partials(m: torch.Tensor, l: torch.Tensor, acc: torch.Tensor) -> Tup
     _require_device(m)
     S, lead, D = m.shape[0], m.shape[1:], acc.shape[-1]
     N = m[0].numel()
-    m32, l32 = m.to(torch.float32).contiguous(), l.to(torch.float32).contiguous()
-    a32 = acc.to(torch.float32).contiguous()
+    m32, l32, a32 = _f32(m), _f32(l), _f32(acc)
     O = torch.empty(N, D, dtype=torch.float32, device=m.device)
     lse = torch.empty(N, dtype=torch.float32, device=m.device)
     lib = _lib.load()
