@@ -176,7 +176,10 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
   const int vt_end = (int)((int64_t)(split + 1) * p.n_vt / n_split);
   const T* Ep = static_cast<const T*>(p.Ep);
 
-  float m[FT], sh[FT], l[FT];  // running maximum, the shift l and acc are relative to
+  // P relative to its tile's maximum: not in fp32, which does not round it, nor in the e4m3 forward, whose
+  // operands are rounded far more coarsely (0.8% faster there)
+  constexpr bool TS = !F8 && sizeof(T) == 2;
+  float m[FT], sh[FT], l[FT];  // running maximum, which l is relative to; the shift acc is relative to
   f32x16_t oacc[DB][FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
@@ -275,15 +278,11 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
       const float mt = wave_max32(mx[ft]), mnew = fmaxf(m[ft], mt);
-      // the e4m3 forward, whose operands are rounded far more coarsely, keeps the running maximum
-      // (0.8% faster there)
-      const float snew = F8 ? mnew : fmaxf(mt, mnew - kShiftBelow);
+      const float snew = TS ? fmaxf(mt, mnew - kShiftBelow) : mnew;
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
-      const float alpha = fast_exp((F8 ? m[ft] : sh[ft]) - shift);  // at most e^kShiftBelow
-      m[ft] = mnew;
-      if (!F8) sh[ft] = snew;
+      const float alpha = fast_exp((TS ? sh[ft] : m[ft]) - shift);  // at most e^kShiftBelow
       float rs = 0.f;
 #pragma unroll
       for (int fv = 0; fv < FV; ++fv)
@@ -293,7 +292,10 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
           sacc[fv][ft][r] = pv;
           rs += pv;
         }
-      l[ft] = l[ft] * alpha + wave_sum32(rs);
+      rs = wave_sum32(rs);
+      l[ft] = TS ? shifted_sum(l[ft], m[ft], rs, shift, mnew) : l[ft] * alpha + rs;
+      m[ft] = mnew;
+      if (TS) sh[ft] = snew;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -343,11 +345,11 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
   for (int ft = 0; ft < FT; ++ft) {
     const int n = n0 + wt * WTR + ft * 32 + (ln & 31);
     // to the running maximum; no score yet: 0
-    const float f = F8 ? 1.f : m[ft] == kNegInf ? 0.f : fast_exp(sh[ft] - m[ft]);
+    const float f = !TS ? 1.f : m[ft] == kNegInf ? 0.f : fast_exp(sh[ft] - m[ft]);
     if (n < ntok) {
       if (ln < 32) {
         p.part_m[(int64_t)part * ntok + n] = m[ft];
-        p.part_l[(int64_t)part * ntok + n] = l[ft] * f;
+        p.part_l[(int64_t)part * ntok + n] = l[ft];
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -414,7 +416,7 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
   const int vt_end = (int)((int64_t)(split + 1) * p.n_vt / n_split);
   const T* Ep = static_cast<const T*>(p.Ep);
 
-  float m[FT], sh[FT], l[FT];  // running maximum, the shift l and acc are relative to
+  float m[FT], sh[FT], l[FT];  // running maximum, which l is relative to; the shift acc is relative to
   f32x16_t oacc[DB][FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
@@ -526,9 +528,8 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
       }
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
-      const float mt = wave_max32(mx[ft]);
-      m[ft] = fmaxf(m[ft], mt);
-      const float snew = fmaxf(mt, m[ft] - kShiftBelow);
+      const float mt = wave_max32(mx[ft]), mnew = fmaxf(m[ft], mt);
+      const float snew = fmaxf(mt, mnew - kShiftBelow);
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
@@ -543,7 +544,8 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
           sacc[fv][ft][r] = pv;
           rs += pv;
         }
-      l[ft] = l[ft] * alpha + wave_sum32(rs);
+      l[ft] = shifted_sum(l[ft], m[ft], wave_sum32(rs), shift, mnew);
+      m[ft] = mnew;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -590,7 +592,7 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
     if (n < ntok) {
       if (ln < 32) {
         p.part_m[(int64_t)part * ntok + n] = m[ft];
-        p.part_l[(int64_t)part * ntok + n] = l[ft] * f;
+        p.part_l[(int64_t)part * ntok + n] = l[ft];
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db)

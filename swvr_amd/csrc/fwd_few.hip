@@ -19,9 +19,9 @@
 //     allow, so 48 to 100 KB of W are in flight per CU: the loop is bound by HBM.
 //     Rows past the run are not loaded;
 //   * the online softmax and acc^T += E^T P^T run as in the general forward,
-//     the tile of 128 rows being each wave's own 32: its maximum, which P's
-//     rounding leaves exact, is the shift of P (O of 1000 tokens on V = 151936 at a
-//     logit spread of 3: 5.8e-5 from 64 bits in bf16, 1.3e-4 with running maxima).
+//     the tile of 128 rows being each wave's own 32: in the 2-byte types its maximum,
+//     which P's rounding leaves exact, is the shift of P (O of 1000 tokens on V = 151936
+//     at a logit spread of 3: 5.8e-5 from 64 bits in bf16, 1.3e-4 with running maxima).
 //     The E^T operand is read from the row-major E tile with transposing LDS reads;
 //   * the waves' partial softmaxes are merged in LDS, so a workgroup writes one
 //     partial; fwd_combine_kernel merges those in a fixed order.
@@ -110,8 +110,8 @@ struct FewCfg {
   static constexpr int NS = FIT < 8 ? FIT : 8;
   static_assert(NS >= 2 && (NS - 2) * L < 64, "ring depth");
   static constexpr int LDS = NS * SB + TE::BYTES;
-  // the merge of the waves' partials reuses the LDS: 4 x [DP][32] floats, then 4 x [32 NB] of three
-  static_assert(kFewWV * (DP * 32 + 3 * 32 * NB) * 4 <= LDS, "merge fits");
+  // the merge of the waves' partials reuses the LDS: 4 x [DP][32] floats, then 4 x [32 NB] of two
+  static_assert(kFewWV * (DP * 32 + 2 * 32 * NB) * 4 <= LDS, "merge fits");
 };
 
 // At most min(ahead, MAX) stages of L loads may stay outstanding.
@@ -201,8 +201,10 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue_next();
 
-  // running maximum, and the shift that l and acc are relative to
-  float m[FT], sh[FT], l[FT];
+  // fp32 keeps the running maximum: it does not round P, and a shift per tile would round l and acc at every
+  // tile instead (8192 tokens on V = 151936: l 3.4e-7 from 64 bits then, 8.4e-8 so)
+  constexpr bool TS = sizeof(T) == 2;
+  float m[FT], sh[FT], l[FT];  // running maximum, which l is relative to; the shift acc is relative to
   f32x16_t oacc[DB][FT], sacc[FT];
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft) {
@@ -276,8 +278,8 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
         mx = fmaxf(mx, x);
       }
       mx = wave_max32(mx);
-      m[ft] = fmaxf(m[ft], mx);
-      const float snew = fmaxf(mx, m[ft] - kShiftBelow);
+      const float mnew = fmaxf(m[ft], mx);
+      const float snew = TS ? fmaxf(mx, mnew - kShiftBelow) : mnew;
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
@@ -290,7 +292,9 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
         sacc[ft][r] = pv;
         rs += pv;
       }
-      l[ft] = l[ft] * alpha + wave_sum32(rs);
+      rs = wave_sum32(rs);
+      l[ft] = TS ? shifted_sum(l[ft], m[ft], rs, shift, mnew) : l[ft] * alpha + rs;
+      m[ft] = mnew;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -320,14 +324,12 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
   float* const sA = reinterpret_cast<float*>(smem);  // [4][DP][32]
   float* const sM = sA + kFewWV * DP * 32;           // [4][32 NB]
   float* const sL = sM + kFewWV * 32 * NB;           // [4][32 NB]
-  float* const sS = sL + kFewWV * 32 * NB;           // [4][32 NB]
 #pragma unroll
   for (int ft = 0; ft < FT; ++ft)
     if (lane < 32) {
       const int c = (wt * FT + ft) * 32 + lane;
       sM[wv * 32 * NB + c] = m[ft];
       sL[wv * 32 * NB + c] = l[ft];
-      sS[wv * 32 * NB + c] = sh[ft];
     }
   __syncthreads();
   for (int bt = 0; bt < WT; ++bt)
@@ -339,7 +341,7 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       for (int j = 0; j < kFewWV; ++j) M = fmaxf(M, sM[j * 32 * NB + c]);
       const float shift = M == kNegInf ? 0.f : M;
       if (wt == bt) {
-        const float f = fast_exp(sh[ft] - shift);  // exp(-inf) = 0: a wave of masked rows adds nothing
+        const float f = expf(sh[ft] - shift);  // exp(-inf) = 0: a wave of masked rows adds nothing
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -355,7 +357,7 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       if (w == 0 && lane < 32 && n0 + c < ntok) {
         float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < kFewWV; ++j) sum += sL[j * 32 * NB + c] * fast_exp(sS[j * 32 * NB + c] - shift);
+        for (int j = 0; j < kFewWV; ++j) sum += sL[j * 32 * NB + c] * expf(sM[j * 32 * NB + c] - shift);
         p.part_m[(int64_t)split * ntok + n0 + c] = M;
         p.part_l[(int64_t)split * ntok + n0 + c] = sum;
       }
