@@ -70,9 +70,15 @@ __device__ __forceinline__ f32x16_t zero16() {
 // exp(x) as 2^(x*log2 e) on the hardware exp2 (v_exp_f32).  exp(-inf) = 0.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
-// Shift of P = e^(s - shift) in the 2-byte forwards: a vocabulary tile's own maximum, but at most this
-// far below the running one (which bounds P's sums).
-constexpr float kShiftBelow = 8.f;
+// Shift of P = e^(s - shift) in the 2-byte forwards, for a vocabulary tile whose largest score is mt and a
+// running maximum m >= mt: the smallest mt + k ln 2 (k whole, up to kShiftSteps) that is not below m, so the
+// tile's largest P is 2^-k, which no rounding to 16 bits changes, and the accumulators are at most what the
+// running maximum itself would make them.  (A shift below m grows them: with 8 below, E of 1e36 in bf16
+// overflowed.)  Tiles further down, and ones of -inf only, take m.
+constexpr float kShiftSteps = 16.f, kLn2 = 0.69314718056f;
+__device__ __forceinline__ float tile_shift(float mt, float m) {
+  return fmaxf(fmaf(fminf(ceilf((m - mt) * kLog2e), kShiftSteps), kLn2, mt), m);
+}
 
 // The running sum l, relative to the running maximum m, after a tile whose sum rs is relative to shift;
 // mnew: the maximum with the tile.  l is scaled only when the maximum rises: carried at each tile's own

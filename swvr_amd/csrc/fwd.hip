@@ -18,9 +18,9 @@
 //     (an independent partial softmax), and P, rounded to the compute dtype as
 //     the reference rounds it (swvr/chunked.py:103, triton_kernels.py:69),
 //     feeds acc^T += E^T P^T straight from the score registers;
-//     P is relative to the tile's own maximum (within 8 of the running one), not
-//     the running maximum: the maximum's row has P = 1, which no rounding
-//     changes, so most rows that dominate a peaked softmax stay exact (O of 3000
+//     P is relative to the tile's own maximum times a power of two (tile_shift), not
+//     to the running maximum: the maximum's row has a P of 1, 1/2, 1/4 ..., which no
+//     rounding changes, so most rows that dominate a peaked softmax stay exact (O of 3000
 //     tokens on V = 151936 at a logit spread of 3: 1.0e-4 from 64 bits in bf16,
 //     1.7e-4 with the running maximum), whatever the number of splits;
 //   * partials (m, l, acc) of all waves and splits are merged by
@@ -278,11 +278,11 @@ __global__ __launch_bounds__((FwdCfg<T, DP, F8>::NT)) void fwd_tile_kernel(FwdPa
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
       const float mt = wave_max32(mx[ft]), mnew = fmaxf(m[ft], mt);
-      const float snew = TS ? fmaxf(mt, mnew - kShiftBelow) : mnew;
+      const float snew = TS ? tile_shift(mt, mnew) : mnew;
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
-      const float alpha = fast_exp((TS ? sh[ft] : m[ft]) - shift);  // at most e^kShiftBelow
+      const float alpha = fast_exp((TS ? sh[ft] : m[ft]) - shift);
       float rs = 0.f;
 #pragma unroll
       for (int fv = 0; fv < FV; ++fv)
@@ -529,11 +529,11 @@ __global__ __launch_bounds__((FwdTile<T, DP>::NT)) void fwd_stream_kernel(FwdPar
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
       const float mt = wave_max32(mx[ft]), mnew = fmaxf(m[ft], mt);
-      const float snew = fmaxf(mt, mnew - kShiftBelow);
+      const float snew = tile_shift(mt, mnew);
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
-      const float alpha = fast_exp(sh[ft] - shift);  // at most e^kShiftBelow
+      const float alpha = fast_exp(sh[ft] - shift);
       sh[ft] = snew;
       float rs = 0.f;
 #pragma unroll

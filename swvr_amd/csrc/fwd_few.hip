@@ -19,9 +19,10 @@
 //     allow, so 48 to 100 KB of W are in flight per CU: the loop is bound by HBM.
 //     Rows past the run are not loaded;
 //   * the online softmax and acc^T += E^T P^T run as in the general forward,
-//     the tile of 128 rows being each wave's own 32: in the 2-byte types its maximum,
-//     which P's rounding leaves exact, is the shift of P (O of 1000 tokens on V = 151936
-//     at a logit spread of 3: 5.8e-5 from 64 bits in bf16, 1.3e-4 with running maxima).
+//     the tile of 128 rows being each wave's own 32, to whose maximum P is relative in
+//     the 2-byte types, times a power of two (tile_shift): its largest P stays exact (O of
+//     1000 tokens on V = 151936 at a logit spread of 3: 5.8e-5 from 64 bits in bf16, 1.3e-4
+//     with running maxima).
 //     The E^T operand is read from the row-major E tile with transposing LDS reads;
 //   * the waves' partial softmaxes are merged in LDS, so a workgroup writes one
 //     partial; fwd_combine_kernel merges those in a fixed order.
@@ -279,11 +280,11 @@ __global__ __launch_bounds__((FewCfg<T, WS, DP, FT, WT>::NT)) void fwd_few_kerne
       }
       mx = wave_max32(mx);
       const float mnew = fmaxf(m[ft], mx);
-      const float snew = TS ? fmaxf(mx, mnew - kShiftBelow) : mnew;
+      const float snew = TS ? tile_shift(mx, mnew) : mnew;
       // a column whose scores so far are all -inf keeps -inf; shift it by 0
       // (swvr/chunked.py:98-99)
       const float shift = snew == kNegInf ? 0.f : snew;
-      const float alpha = fast_exp(sh[ft] - shift);  // at most e^kShiftBelow
+      const float alpha = fast_exp(sh[ft] - shift);
       sh[ft] = snew;
       float rs = 0.f;
 #pragma unroll

@@ -44,3 +44,33 @@ def test_sums_over_a_long_vocabulary(dtype, N, D):
     print(f"\n{dtype} {N}: l {e_l:.2e} lse {e_lse:.2e} O {e_O:.2e}")
     assert e_l <= 2 ** -23 and e_lse <= 2 ** -23 and e_O <= {torch.float32: 4e-6, torch.bfloat16: 1.2e-3,
                                                          torch.float16: 1.5e-4}[dtype]
+
+
+# E near the largest finite values under scores that fall by 20 after the first row and, in the middle, rise
+# again: no accumulator may pass what P <= 1 makes of them.  Vocabularies of several tiles per workgroup.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,V,D", [(40, 140001, 64), (700, 70001, 100), (1000, 20000, 64), (1000, 20000, 128),
+                                   (1000, 20000, 256), (1000, 20000, 300)])
+def test_embeddings_near_the_largest_finite_values(dtype, N, V, D):
+    h, W = torch.zeros(N, 16, device="cuda", dtype=dtype), torch.zeros(V, 16, device="cuda", dtype=dtype)
+    b = torch.zeros(V, device="cuda")
+    b[0], b[V // 2], b[V // 2 + 1:V // 2 + 300] = 20, 15, -9
+    E = torch.full((V, D), 2.0 ** 125, device="cuda", dtype=dtype)
+    E[1::2] *= -1
+    O, lse = swvr.softmax_readout(h, W, E, b)
+    want_O, want_lse = readout64(h, W, E, b)
+    assert rel_err(O, want_O) <= 1e-3 and rel_err(lse, want_lse) <= 1e-6
+
+
+# scores that rise and fall by 40 over the vocabulary: shifts above, below and far below the running maximum
+@pytest.mark.parametrize("dtype,bar", [(torch.bfloat16, 1e-3), (torch.float16, 2e-4), (torch.float32, 3e-6)])
+@pytest.mark.parametrize("N,V,D,waves", [(3, 9001, 64, 3), (300, 40001, 33, 50), (700, 9001, 200, 7), (1500, 40001, 64, 40),
+                                         (1500, 40001, 128, 40), (1500, 40001, 300, 9)])
+def test_scores_that_rise_and_fall(dtype, bar, N, V, D, waves):
+    h, W, E, _ = exact_scores(N, 64, V, D, dtype)
+    b = 20 * torch.sin(torch.arange(V, device="cuda") * (2 * torch.pi * waves / V))
+    O, lse = swvr.softmax_readout(h, W, E, b)
+    want_O, want_lse = readout64(h, W, E, b)
+    e_O, e_lse = rel_err(O, want_O), rel_err(lse, want_lse)
+    print(f"\n{dtype} {N} {V} {D}: O {e_O:.2e} lse {e_lse:.2e}")
+    assert e_O <= bar and e_lse <= 2 ** -23
