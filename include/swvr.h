@@ -147,11 +147,19 @@ int swvr_combine(int64_t S, int64_t N, int64_t D, const float* m, const float* l
 
 /* Workspace bytes swvr_bwd needs.  `chunk` is the vocabulary staging chunk
  * (the reference's chunk_size, swvr/chunked.py:120): the backward stages
- * dS for `chunk` vocabulary rows at a time, so this is O(N * chunk).  Fewer
- * than 8192 tokens stage several chunks of 8192 rows or more together, up to
- * the memory 8192 tokens would take (swvr_bwd_tiling reports the rows). */
+ * dS for `chunk` vocabulary rows (rounded up to its tiles) at a time, so this
+ * is O((N + K) * chunk) beyond the packed E and h. */
 size_t swvr_bwd_workspace_size(int dtype, int64_t N, int64_t K, int64_t V, int64_t D,
                                int64_t chunk, int need_gh);
+
+/* A chunk for callers that name none: 8192 rows, or with up to 4096 tokens 2,
+ * 4, 8 ... times as many, which takes fewer launches, as long as the workspace
+ * stays within the one that 8192 tokens need at 8192 rows, but for up to 64 MB
+ * of further partial sums of gh.  K8: bytes per row of the e4m3 operands
+ * (swvr_bwd_fp8), else 0; w_dtype as in swvr_bwd_mixed.  0 for bad sizes.
+ * No reference counterpart. */
+int64_t swvr_bwd_default_chunk(int dtype, int w_dtype, int64_t N, int64_t K, int64_t K8,
+                               int64_t V, int64_t D, int need_gh);
 
 /* Backward.  Replaces swvr::chunked_bwd (swvr/chunked.py:170-178, 108-151).
  * Inputs: the forward's operands, O [N,D] fp32 (row stride D), lse [N] fp32,
@@ -204,7 +212,7 @@ int swvr_bwd_f64(int64_t N, int64_t K, int64_t V, int64_t D, const double* h, in
  * scores kernel; [1] BV, its vocabulary tile; [2] G, the token groups a
  * vocabulary tile's token blocks are split over (one workgroup per group, so a
  * workgroup walks ceil(active token blocks / G) blocks); [3] C, the vocabulary
- * rows staged together (a chunk, or several with few tokens); [4] how many such; [5] DP, the padded embedding
+ * rows per chunk; [4] the number of chunks; [5] DP, the padded embedding
  * width; [6] the scores kernel: 1 the narrow-embedding kernel (side tiles
  * carried by its K ring), 2 the wide-embedding kernel (gO and E streamed as
  * D-slices; dE formed by the gradient GEMM launch), 0 the general one.

@@ -91,6 +91,16 @@ def _lead_stride(x):
     return x.stride(0) if x.shape[0] > 1 else x.shape[1]
 
 
+def _rows_staged(chunk, tag, w_tag, N, K, V, D, need_h, K8=0):
+    """Vocabulary rows the backward stages at a time: the caller's ``chunk``, or for None the library's
+    choice for these sizes (swvr_bwd_default_chunk, 8192 where the first test says so)."""
+    if chunk is None and (N > 4096 or V <= DEFAULT_CHUNK):
+        chunk = DEFAULT_CHUNK
+    if chunk is None:
+        chunk = _lib.load().swvr_bwd_default_chunk(tag, w_tag, N, K, K8, V, D, int(need_h)) or DEFAULT_CHUNK
+    return int(chunk)
+
+
 def _f64(x):
     """``x`` in fp64 with unit stride in its last dimension (or None)."""
     if x is None:
@@ -145,7 +155,7 @@ def _backward_f64(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, need_h, n
 def _forward(h, W, E, bias, logit_scale, chunk, cdt):
     _require_device(h)
     if cdt == torch.float64:
-        return _forward_f64(h, W, E, bias, logit_scale, chunk)
+        return _forward_f64(h, W, E, bias, logit_scale, chunk or DEFAULT_CHUNK)
     lib = _lib.load()
     if cdt not in _lib.DTYPE_TAG:
         raise NotImplementedError(f"swvr_amd: compute dtype {cdt} is not supported (bf16, fp16, fp32, fp64)")
@@ -204,7 +214,8 @@ def _grad_buffer(shape, want, device):
 def _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, need_h, need_W, need_E, need_b):
     _require_device(h)
     if cdt == torch.float64:
-        return _backward_f64(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, need_h, need_W, need_E, need_b)
+        return _backward_f64(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk or DEFAULT_CHUNK, need_h, need_W,
+                             need_E, need_b)
     lib = _lib.load()
     N, K = h.shape
     V, D = E.shape
@@ -218,7 +229,8 @@ def _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, need_h, 
     gb = torch.empty(V, dtype=torch.float32, device=dev) if need_b else None
     gO32, glse32, O32, lse32 = _f32(gO), _f32(glse), _f32(O), _f32(lse)
     tag = _lib.DTYPE_TAG[cdt]
-    ws_bytes = lib.swvr_bwd_workspace_size_mixed(tag, w_tag, N, Kp, V, D, int(chunk), int(need_h))
+    chunk = _rows_staged(chunk, tag, w_tag, N, Kp, V, D, need_h)
+    ws_bytes = lib.swvr_bwd_workspace_size_mixed(tag, w_tag, N, Kp, V, D, chunk, int(need_h))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
 
     def tag_of(t):
@@ -227,7 +239,7 @@ def _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, need_h, 
     with torch.cuda.device(dev):
         rc = lib.swvr_bwd_mixed(tag, h_tag, w_tag, N, Kp, V, D, _lib.ptr(hc), _lead_stride(hc), _lib.ptr(Wc),
                                 _lead_stride(Wc), _lib.ptr(Ec), _lead_stride(Ec), _lib.ptr(b), float(logit_scale),
-                                _lib.ptr(O32), _lib.ptr(lse32), _lib.ptr(gO32), _lib.ptr(glse32), int(chunk),
+                                _lib.ptr(O32), _lib.ptr(lse32), _lib.ptr(gO32), _lib.ptr(glse32), chunk,
                                 _lib.ptr(gh), tag_of(gh), _lib.ptr(gW), tag_of(gW), _lib.ptr(gE), tag_of(gE),
                                 _lib.ptr(gb), _lib.ptr(ws), ws_bytes, _lib.stream_of(dev))
     _lib.check(rc)
@@ -404,16 +416,16 @@ def readout_mse_eager(h2, W, E, bias, target2, weight, active, z, reduction, log
     red = REDUCTIONS[reduction]
     if _needs_grad(h2, W, E, bias):
         return _ReadoutMse.apply(h2, W, E, bias, target2, weight, active, float(z), red, float(logit_scale),
-                                 int(chunk), cdt)
+                                 chunk, cdt)
     if active:
-        O, lse = _forward_active(h2, W, E, bias, weight, float(logit_scale), int(chunk), cdt)
+        O, lse = _forward_active(h2, W, E, bias, weight, float(logit_scale), chunk, cdt)
     else:
-        O, lse = _forward(h2, W, E, bias, float(logit_scale), int(chunk), cdt)
+        O, lse = _forward(h2, W, E, bias, float(logit_scale), chunk, cdt)
     return _mse_loss(O, lse, target2, weight, float(z), red, False)[0]
 
 
 def _readout_eager(h2, W, E, bias, weight, logit_scale, chunk, cdt):
-    args = (float(logit_scale), int(chunk), cdt)
+    args = (float(logit_scale), chunk, cdt)
     if _needs_grad(h2, W, E, bias):
         return _Readout.apply(h2, W, E, bias, weight, *args)
     if weight is None:
@@ -422,9 +434,11 @@ def _readout_eager(h2, W, E, bias, weight, logit_scale, chunk, cdt):
 
 
 def softmax_readout_op(h2, W, E, bias, logit_scale, chunk, cdt):
-    """``h2`` is ``[N, K]``; returns ``(O [N, D], LSE [N])`` in fp32 (swvr/chunked.py:208-212)."""
+    """``h2`` is ``[N, K]``; returns ``(O [N, D], LSE [N])`` in fp32 (swvr/chunked.py:208-212).  ``chunk``
+    None: the library's choice on an eager call; the ops, whose sizes may be symbols, take 8192."""
     if eager(h2, W, E, bias):
         return _readout_eager(h2, W, E, bias, None, logit_scale, chunk, cdt)
+    chunk = chunk or DEFAULT_CHUNK
     if h2.device.type not in ("cuda", "cpu"):  # meta / fake tracing: no autocast state
         return _fwd_op(h2, W, E, bias, float(logit_scale), int(chunk), cdt, True)
     with torch.autocast(h2.device.type, enabled=False):
@@ -436,6 +450,7 @@ def softmax_readout_active_op(h2, W, E, bias, weight, logit_scale, chunk, cdt):
     of 0 instead of their readout (``swvr_fwd_active``); ``weight`` is [N], no gradient."""
     if eager(h2, W, E, bias, weight):
         return _readout_eager(h2, W, E, bias, weight, logit_scale, chunk, cdt)
+    chunk = chunk or DEFAULT_CHUNK
     if h2.device.type not in ("cuda", "cpu"):
         return _fwd_active_op(h2, W, E, bias, weight, float(logit_scale), int(chunk), cdt)
     with torch.autocast(h2.device.type, enabled=False):

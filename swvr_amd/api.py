@@ -21,6 +21,15 @@ def default_chunk_size():
     return int(raw) if raw else DEFAULT_CHUNK
 
 
+def _chunk(chunk_size):
+    """A call's chunk: ``chunk_size`` or ``SWVR_CHUNK`` where one is given, else None (the library's choice
+    for the sizes)."""
+    chunk = int(chunk_size) if chunk_size else default_chunk_size() if os.environ.get("SWVR_CHUNK") else None
+    if chunk is not None and chunk <= 0:
+        raise ValueError(f"chunk_size must be positive, got {chunk}")
+    return chunk
+
+
 def _compute_dtype(h, W):
     """dtype the products run in: autocast's if it is active on h's device, otherwise the type
     promotion of h and W (swvr/api.py:8-11)."""
@@ -51,16 +60,15 @@ def softmax_readout(h, W, E, bias=None, *, logit_scale=1.0, chunk_size=None):
     h ``[..., K]``, W ``[V, K]``, E ``[V, D]``, optional bias ``[V]``.  O and LSE are fp32,
     or fp64 when the products run in fp64.  The [tokens, V] scores never exist in memory;
     the backward recomputes them ``chunk_size`` rows of the vocabulary at a time (default
-    8192, or ``SWVR_CHUNK``), which bounds its extra memory by O(tokens * chunk_size); fewer
-    than 8192 tokens take several chunks of 8192 or more at a time, within 8192 tokens' memory.
+    8192, or ``SWVR_CHUNK``), which bounds its extra memory by O((tokens + K) * chunk_size).  Where
+    neither is given, eager calls of up to 4096 tokens take 2, 4, 8 ... times 8192 rows at a time, within
+    the memory that 8192 tokens take at 8192 (and up to 64 MB for partial sums of h's gradient).
     Autograd reaches every input that requires a gradient.
     """
     _check(h, W, E, bias)
     lead = h.shape[:-1]
     h2 = _rows(h)
-    chunk = int(chunk_size) if chunk_size else default_chunk_size()
-    if chunk <= 0:
-        raise ValueError(f"chunk_size must be positive, got {chunk}")
+    chunk = _chunk(chunk_size)
     O, lse = softmax_readout_op(h2, W, E, bias, logit_scale, chunk, _compute_dtype(h, W))
     if h2 is h:
         return O, lse
@@ -85,9 +93,7 @@ def softmax_readout_mse(h, W, E, target, bias=None, *, weight=None, reduction="m
     skips = _skips_zero_weight(h, W, weight, reduction)
     if _one_call(h, W, E, target, bias, weight, reduction):
         _check(h, W, E, bias)
-        chunk = int(chunk_size) if chunk_size else default_chunk_size()
-        if chunk <= 0:
-            raise ValueError(f"chunk_size must be positive, got {chunk}")
+        chunk = _chunk(chunk_size)
         out = readout_mse_eager(_rows(h), W, E, bias, _rows(target), weight.reshape(-1) if weight is not None else None,
                                 skips, z_loss_weight, reduction, logit_scale, chunk, _compute_dtype(h, W))
         return out.view(h.shape[:-1]) if reduction == "none" else out
@@ -98,9 +104,7 @@ def softmax_readout_mse(h, W, E, target, bias=None, *, weight=None, reduction="m
         # the reference's NaNs).
         _check(h, W, E, bias)
         lead = h.shape[:-1]
-        chunk = int(chunk_size) if chunk_size else default_chunk_size()
-        if chunk <= 0:
-            raise ValueError(f"chunk_size must be positive, got {chunk}")
+        chunk = _chunk(chunk_size)
         O, lse = softmax_readout_active_op(h.reshape(-1, h.shape[-1]), W, E, bias, weight.reshape(-1),
                                            logit_scale, chunk, _compute_dtype(h, W))
         O, lse = O.view(*lead, E.shape[1]), lse.view(lead)

@@ -320,6 +320,12 @@ size_t swvr_bwd_workspace_size(int dtype, int64_t N, int64_t K, int64_t V, int64
   return swvr_bwd_workspace_size_mixed(dtype, dtype, N, K, V, D, chunk, need_gh);
 }
 
+int64_t swvr_bwd_default_chunk(int dtype, int w_dtype, int64_t N, int64_t K, int64_t K8, int64_t V, int64_t D,
+                               int need_gh) {
+  if (!is_dtype(dtype) || N < 0 || K < 0 || K8 < 0 || V < 0 || D < 0) return 0;
+  return bwd_default_chunk(dtype, N, K, V, D, need_gh != 0, w_dtype != dtype, K8);
+}
+
 int swvr_bwd_tiling(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chunk, int64_t* out, int n_out) {
   g_err[0] = 0;
   if (!out || n_out < 0) return fail(SWVR_EINVAL, "out must be non-null");

@@ -1913,28 +1913,6 @@ hipError_t compact_tokens(const int* flag, int N, int* idx, int* inv, int* n_act
   return hipGetLastError();
 }
 
-// Chunks of the vocabulary that a backward of few tokens stages together.  Each chunk costs a scores
-// and a GEMM launch, which few token blocks leave mostly idle (500 tokens, K = 1024: 64 scores workgroups
-// and 256 short GEMM tiles per 8192 rows), and one more read and write of every dh accumulator.  So
-// fewer than 8192 tokens stage as many rows as 8192 tokens' memory at the given chunk holds, the packed
-// rows of W staying within 256 MB.  A chunk below the default of 8192 rows asks for less memory and is
-// kept as it is.  Powers of two only: 8192 rows are 32 vocabulary tiles, and 3 or 6 such chunks leave a
-// quarter of the CUs without a scores workgroup (1024 tokens, K = 2560, V = 151936: 6 chunks 3.87 ms, 4
-// 3.67).  Steps, one chunk at a time / 4096 tokens' memory / 8192: 500 tokens, K = 1024, V = 32000 (all 4
-// chunks) 418 / 317 / 317 us; 2048 tokens, K = 1024, V = 151936, gradient of h alone 2.60 / 2.26 / 2.15 ms;
-// 1332 in fp32, K = 768, V = 30001 2.65 / 2.39 / 2.29; 1280 tokens, K = 1024, V = 151936 - / 2.16 / 2.03;
-// 4096, K = 1024, V = 128256, gradient of h alone 3.47 / 3.47 / 3.35.  16384 tokens' memory gives up to
-// 3% more at twice the bytes (1280 tokens 1.97 ms, the others within 1%).
-constexpr int64_t kChunkDefault = 8192, kChunkTokens = 8192, kChunkPackBytes = (int64_t)256 << 20;
-int64_t chunks_together(int64_t N_pad, int64_t K, int64_t chunk, int64_t tb) {
-  if (chunk < kChunkDefault || N_pad >= kChunkTokens || chunk > ((int64_t)1 << 22)) return 1;
-  const int64_t by_tokens = kChunkTokens / N_pad, by_pack = kChunkPackBytes / (chunk * (K > 0 ? K : 1) * tb);
-  const int64_t most = by_tokens < by_pack ? by_tokens : by_pack;
-  int64_t n = 1;
-  while (2 * n <= most) n *= 2;
-  return n;
-}
-
 bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chunk, bool need_gh, BwdPlan* plan,
               bool w_f32, int64_t K8) {
   const bool f8 = K8 > 0;
@@ -1987,8 +1965,7 @@ bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chu
   plan->n_tb = (int)((N + BM - 1) / BM);
   plan->N_pad = ((N + 255) / 256) * 256;
   if (plan->N_pad == 0) plan->N_pad = 256;
-  int64_t c = chunk * chunks_together(plan->N_pad, K, chunk, two ? 2 : 4);
-  if (c > V) c = V;
+  int64_t c = chunk < V ? chunk : V;
   // at most 2^22 rows per chunk: tile-relative offsets into [DP or rows][C] buffers stay 32-bit
   if (c > ((int64_t)1 << 22)) c = (int64_t)1 << 22;
   if (c < 1) c = 1;
@@ -2023,8 +2000,10 @@ bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chu
     const int64_t n_n = (K + GN - 1) / GN, sl = two ? SliceK<bf16_t>::value : SliceK<float>::value;
     const int64_t n_dw = (c + GM - 1) / GM * n_n, n_dh = (N + GM - 1) / GM * n_n, acc = N * K * 4;
     const int slots = two ? 256 : 512, o_dw = two ? 8 : 5, o_dh = two ? 12 : 7;
-    plan->dh_split_w = dh_split_of(n_dw, (N + sl - 1) / sl, n_dh, c / sl, slots, o_dw, o_dh, acc);
-    plan->dh_split_h = dh_split_of(0, 0, n_dh, c / sl, slots, o_dw, o_dh, acc);
+    // O(N x chunk) as the rest of the workspace
+    const int64_t stages = 2 * c * plan->N_pad * (int64_t)tb, room = stages < kDhSplitBytes ? stages : kDhSplitBytes;
+    plan->dh_split_w = dh_split_of(n_dw, (N + sl - 1) / sl, n_dh, c / sl, slots, o_dw, o_dh, acc, room);
+    plan->dh_split_h = dh_split_of(0, 0, n_dh, c / sl, slots, o_dw, o_dh, acc, room);
     const int s = plan->dh_split_w > plan->dh_split_h ? plan->dh_split_w : plan->dh_split_h;
     off += align256((size_t)acc * s);
   }
@@ -2068,6 +2047,34 @@ bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chu
   if (K8 > 0) off += align256((size_t)plan->V_pad * 4);
   plan->ws_bytes = off;
   return true;
+}
+
+// Chunks of kChunkDefault rows that a backward whose caller gives no chunk stages together.  Each chunk
+// costs a scores and a GEMM launch, which few token blocks leave mostly idle (500 tokens, K = 1024: 64
+// scores workgroups and 256 short GEMM tiles per 8192 rows), and one more read and write of every dh
+// accumulator.  So up to 4096 tokens stage as many chunks as fit, with everything that is held per row of a
+// chunk (stages, packed and rounded rows of W, dE and db partials), into the workspace that 8192 tokens take
+// at one chunk; the sums of dh's vocabulary runs beyond the first, bounded by kDhSplitBytes, are not counted.
+// Powers of two only: 8192 rows are 32 vocabulary tiles, and 3 or 6 such chunks leave a quarter of the CUs
+// without a scores workgroup (1024 tokens, K = 2560, V = 151936: 6 chunks 3.87 ms, 4 3.67).  Steps, one chunk
+// at a time / in 4096 tokens' memory / in 8192's: 500 tokens, K = 1024, V = 32000 (all 4 chunks) 418 / 317 /
+// 317 us; 2048 tokens, K = 1024, V = 151936, gradient of h alone 2.60 / 2.26 / 2.15 ms; 1332 in fp32,
+// K = 768, V = 30001 2.65 / 2.39 / 2.29; 4096, K = 1024, V = 128256, gradient of h alone 3.47 / 3.47 / 3.35.
+// 16384 tokens' memory gives up to 3% more at twice the bytes.
+constexpr int64_t kChunkDefault = 8192, kChunkTokens = 8192;
+int64_t bwd_default_chunk(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, bool need_gh, bool w_f32, int64_t K8) {
+  BwdPlan plan;
+  // workspace without the further sums of dh's runs
+  auto bytes = [&](int64_t n_tok, int64_t chunk) {
+    if (!bwd_plan(dtype, n_tok, K, V, D, chunk, need_gh, &plan, w_f32, K8)) return SIZE_MAX;
+    return plan.ws_bytes - (plan.off_gO - plan.off_dh) + (need_gh ? (size_t)n_tok * K * 4 : 0);
+  };
+  int64_t n = 1;
+  while (2 * n * ((N + 255) / 256 * 256) <= kChunkTokens && n * kChunkDefault < V) n *= 2;
+  if (N <= 0 || n == 1) return kChunkDefault;
+  const size_t most = bytes(kChunkTokens, kChunkDefault);
+  while (n > 1 && bytes(N, n * kChunkDefault) > most) n /= 2;
+  return n * kChunkDefault;
 }
 
 hipError_t bwd_launch(int dtype, const BwdPlan& plan, const BwdParams& p, hipStream_t stream) {

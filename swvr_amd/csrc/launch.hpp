@@ -216,13 +216,14 @@ inline int de_split(int64_t n_pad) {
 // duration when `slots` workgroups run at a time, dW tiles dealt first, with o_dw / o_dh slices'
 // worth of time per tile for its prologue and stores: a run that ends in a read-modify-write of
 // its accumulator costs more than a dW tile.  Runs keep at least 8 slices, the accumulators beyond
-// the first (acc_bytes each) stay within kDhSplitBytes, and a split must gain 5%.
+// the first (acc_bytes each) stay within `room` (two dS stages and kDhSplitBytes), and a split must
+// gain 5%.
 // Measured, the whole call, whole tiles against split: N = 2048, K = 1024, V = 151936, gh alone (32 dh
 // tiles per chunk, 8 runs) 4.65 -> 2.63 ms; N = 500, K = 1024, V = 32000, every gradient (8 dh and 128
 // dW tiles, 16 runs) 1.02 -> 0.53 ms; N = 2048, K = 2048, V = 65536 (64 and 256, 4 runs) 3.48 -> 2.95.
 constexpr int64_t kDhSplitBytes = (int64_t)64 << 20;
 inline int dh_split_of(int64_t n_dw, int64_t s_dw, int64_t n_dh, int64_t s_dh, int slots, int o_dw, int o_dh,
-                       int64_t acc_bytes) {
+                       int64_t acc_bytes, int64_t room) {
   if (n_dh <= 0) return 1;
   const int64_t a = s_dw + o_dw, q = n_dw / slots, r = n_dw % slots;
   auto span = [&](int64_t s) {
@@ -243,7 +244,7 @@ inline int dh_split_of(int64_t n_dw, int64_t s_dw, int64_t n_dh, int64_t s_dh, i
   };
   int64_t best = span(1) * 95 / 100;
   int split = 1;
-  for (int s = 2; s <= 64 && s_dh / s >= 8 && (s - 1) * acc_bytes <= kDhSplitBytes; s *= 2) {
+  for (int s = 2; s <= 64 && s_dh / s >= 8 && (s - 1) * acc_bytes <= room; s *= 2) {
     const int64_t t = span(s);
     if (t < best) {
       best = t;
@@ -258,6 +259,8 @@ inline int dh_split_of(int64_t n_dw, int64_t s_dw, int64_t n_dh, int64_t s_dh, i
 // K8 > 0: the scores are recomputed from e4m3 h and W of K8 bytes per row.
 bool bwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, int64_t chunk, bool need_gh,
               BwdPlan* plan, bool w_f32 = false, int64_t K8 = 0);
+// Vocabulary rows to stage at a time when the caller names no chunk.
+int64_t bwd_default_chunk(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, bool need_gh, bool w_f32, int64_t K8);
 
 struct BwdParams {
   const void* h;

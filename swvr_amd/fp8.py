@@ -23,7 +23,7 @@ h and W (the quantisation passes gradients through as the identity).
 import torch
 
 from . import _lib
-from ._ops import _embed, _f32, _grad_buffer, _kpad, _lead_stride, _matrix, _plain, _require_device
+from ._ops import _embed, _f32, _grad_buffer, _kpad, _lead_stride, _matrix, _plain, _require_device, _rows_staged
 
 E4M3 = torch.float8_e4m3fn
 E4M3_MAX = 448.0
@@ -108,7 +108,8 @@ def _bwd(gO, glse, h, W, E, bias, O, lse, hq, hs, Wq, ws, logit_scale, chunk, ne
     gb = torch.empty(V, dtype=torch.float32, device=dev) if need_b else None
     gO32, glse32 = _f32(gO), _f32(glse)
     Kq = hq.shape[1]
-    ws_bytes = lib.swvr_bwd_fp8_workspace_size(N, Kp, Kq, V, D, int(chunk), int(need_h))
+    chunk = _rows_staged(chunk, _lib.BF16, _lib.BF16, N, Kp, V, D, need_h, Kq)
+    ws_bytes = lib.swvr_bwd_fp8_workspace_size(N, Kp, Kq, V, D, chunk, int(need_h))
     work = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
 
     def tag_of(t):
@@ -119,7 +120,7 @@ def _bwd(gO, glse, h, W, E, bias, O, lse, hq, hs, Wq, ws, logit_scale, chunk, ne
         rc = lib.swvr_bwd_fp8(N, Kp, V, D, _lib.ptr(hb), _lead_stride(hb), _lib.ptr(Wb), _lead_stride(Wb),
                               _lib.ptr(Eb), lde, _lib.ptr(b), float(logit_scale), _lib.ptr(hq), Kq, Kq,
                               _lib.ptr(hs), _lib.ptr(Wq), Kq, _lib.ptr(ws), _lib.ptr(O), _lib.ptr(lse),
-                              _lib.ptr(gO32), _lib.ptr(glse32), int(chunk), _lib.ptr(gh), tag_of(gh), _lib.ptr(gW),
+                              _lib.ptr(gO32), _lib.ptr(glse32), chunk, _lib.ptr(gh), tag_of(gh), _lib.ptr(gW),
                               tag_of(gW), _lib.ptr(gE), tag_of(gE), _lib.ptr(gb), _lib.ptr(work), ws_bytes,
                               _lib.stream_of(dev))
     _lib.check(rc)
@@ -164,10 +165,10 @@ def softmax_readout_fp8(h, W, E, bias=None, *, logit_scale=1.0, w_q=None, chunk_
     Shapes as ``softmax_readout``: h ``[..., K]``, W ``[V, K]``, E ``[V, D]`` (D <= 128),
     bias ``[V]``.  ``w_q`` = ``quantize_rows(W)`` reuses a quantised W across calls (W is
     then only used for its shape, and for the gradient products).  Differentiable: the
-    backward recomputes the same e4m3 scores and stages ``chunk_size`` (default 8192)
-    vocabulary rows of dS at a time; gh, gW, gE and gb come out in the parameters' dtypes.
+    backward recomputes the same e4m3 scores and stages ``chunk_size`` (default
+    as ``softmax_readout``'s) vocabulary rows of dS at a time; gh, gW, gE and gb come out in the parameters' dtypes.
     """
-    from .api import _check, default_chunk_size
+    from .api import _check, _chunk
     _check(h, W, E, bias)
     _require_device(h)
     lead = h.shape[:-1]
@@ -180,9 +181,7 @@ def softmax_readout_fp8(h, W, E, bias=None, *, logit_scale=1.0, w_q=None, chunk_
     # the kernels read dense rows of Kp bytes and fp32 scales
     Wq = Wq.contiguous()
     ws = _f32(ws.to(device=h.device))
-    chunk = int(chunk_size) if chunk_size else default_chunk_size()
-    if chunk <= 0:
-        raise ValueError(f"chunk_size must be positive, got {chunk}")
+    chunk = _chunk(chunk_size)
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (h, W, E, bias)):
         O, lse = _Fp8Readout.apply(h2, W, E, bias, float(logit_scale), chunk, hq, hs, Wq, ws)
     else:

@@ -25,7 +25,7 @@ import torch
 
 from . import _lib
 from ._ops import _backward, _embed, _f32, _kpad, _lead_stride, _matrix, _require_device
-from .api import _check, _compute_dtype, default_chunk_size
+from .api import _check, _chunk, _compute_dtype
 
 
 def softmax_readout_partial(h: torch.Tensor, W: torch.Tensor, E: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -95,9 +95,7 @@ def shard_backward(gO: torch.Tensor, glse: torch.Tensor, h: torch.Tensor, W: tor
     lead = h.shape[:-1]
     h2 = h.reshape(-1, h.shape[-1])
     N, D = h2.shape[0], E.shape[1]
-    chunk = int(chunk_size) if chunk_size else default_chunk_size()
-    if chunk <= 0:
-        raise ValueError(f"chunk_size must be positive, got {chunk}")
+    chunk = _chunk(chunk_size)
     need_h, need_W, need_E, need_b = need
     gh, gW, gE, gb = _backward(gO.reshape(N, D), glse.reshape(N), h2, W, E, bias, O.reshape(N, D), lse.reshape(N),
                                logit_scale, chunk, cdt, need_h, need_W, need_E, need_b and bias is not None)

@@ -219,10 +219,31 @@ def test_active_positions_on_the_few_token_kernel(dtype, N, count, V, D):
     assert O.isnan().all() and lse.isnan().all()
 
 
-# several chunks staged together, and a second such group that is not whole
-@pytest.mark.parametrize("dtype,N,K,V,D", [(torch.bfloat16, 200, 64, 140001, 24), (torch.bfloat16, 1030, 72, 40000, 100),
-                                           (torch.float32, 520, 64, 66000, 16)])
+# no chunk given: several times 8192 rows staged together, and a second such group that is not whole
+@pytest.mark.parametrize("dtype,N,K,V,D", [(torch.bfloat16, 200, 64, 270001, 24),
+                                           (torch.bfloat16, 1030, 72, 40000, 100), (torch.float32, 520, 64, 66000, 16)])
 def test_chunks_staged_together(dtype, N, K, V, D):
     inputs = make(N, K, V, D, dtype, w_scale=1.0)
     bars = (1e-2, 2e-2) if dtype == torch.bfloat16 else (1e-5, 1e-5)
-    check(inputs, lambda *a: swvr.softmax_readout(*a, chunk_size=8192), (N,), D, *bars)
+    from swvr_amd import _lib, _ops
+    tag = _lib.DTYPE_TAG[dtype]
+    rows = _ops._rows_staged(None, tag, tag, N, (K + 7) // 8 * 8, V, D, True)
+    assert 8192 < rows < V
+    check(inputs, swvr.softmax_readout, (N,), D, *bars)
+
+
+@pytest.mark.parametrize("chunk", [8192, None])
+def test_backward_memory_of_few_tokens(chunk):
+    """Beyond the gradients: a given chunk's workspace (69 MiB here), or without one at most what 8192 tokens
+    take at 8192 rows (294 MiB) and 64 MiB; 10 MiB for the rest of the call."""
+    N, K, V, D = 500, 1024, 151936, 64
+    xs = make(N, K, V, D, torch.bfloat16)
+    loss = swvr.softmax_readout_mse(*xs[:3], torch.randn(N, D, device="cuda"), xs[3], chunk_size=chunk)
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    grads = torch.autograd.grad(loss, xs)
+    torch.cuda.synchronize()
+    extra = (torch.cuda.max_memory_allocated() - base - sum(g.numel() * g.element_size() for g in grads)) / 2**20
+    print(f"{extra:.0f} MiB")
+    assert extra <= (69 if chunk else 294 + 64) + 10
