@@ -43,13 +43,17 @@ def _plain(x):
     """``x`` with its values in memory as they are read by pointer: autograd hands out, and callers may
     pass, views whose sign is still to be flipped (``z.conj().imag``) and zeros without memory, which only
     the dispatcher resolves; ``.to`` and ``.contiguous()`` return such a one-element view as it is."""
-    x = x.resolve_neg()
+    if x.is_neg():
+        x = x.resolve_neg()
     return x.clone() if x._is_zerotensor() else x
 
 
 def _f32(x):
     """``x`` as a dense fp32 tensor (or None)."""
-    return None if x is None else _plain(x).to(torch.float32).contiguous()
+    if x is None:
+        return None
+    x = _plain(x)
+    return (x if x.dtype == torch.float32 else x.to(torch.float32)).contiguous()
 
 
 def _matrix(x, cdt, Kp):
@@ -343,8 +347,10 @@ def eager(*tensors):
             or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0):
         return False
-    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and t.device.type == "cuda")
-               for t in tensors)
+    for t in tensors:  # (a loop: 4 us less per call than a generator)
+        if t is not None and not (t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter)):
+            return False
+    return True
 
 
 def _needs_grad(*tensors):
@@ -358,12 +364,16 @@ def _save(ctx, tensors, args):
 
 
 def _readout_grads(ctx, gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt):
-    """The four gradients, None where not needed (as ``_autograd_backward``)."""
+    """The four gradients, None where not needed (as ``_autograd_backward``): through swvr::chunked_bwd where
+    something looks at the ops while the backward runs, whatever the forward saw."""
     needs = [bool(n) for n in ctx.needs_input_grad[:4]]
     needs[3] = needs[3] and bias is not None
     gO = gO if gO is not None else torch.zeros_like(O)
     glse = glse if glse is not None else torch.zeros_like(lse)
-    return _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, *needs)
+    if eager(gO, glse, h, W, E, bias, O, lse):
+        return _backward(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk, cdt, *needs)
+    grads = _bwd_op(gO, glse, h, W, E, bias, O, lse, logit_scale, chunk or DEFAULT_CHUNK, cdt, True, *needs)
+    return [g if need else None for g, need in zip(grads, needs)]
 
 
 class _Readout(torch.autograd.Function):

@@ -89,6 +89,26 @@ def test_whatever_looks_at_the_ops_sees_them():
         assert not _ops.eager(xs[0])
 
 
+@pytest.mark.parametrize("loss", ["readout", "mse", "weighted"])
+def test_a_backward_run_under_a_mode_shows_its_op(loss):
+    xs = make(20, 64, 300, 16, torch.float32)
+    xs[1].requires_grad_(False)
+    target, weight = torch.randn(20, 16, device="cuda"), (torch.arange(20, device="cuda") % 4 > 0).float()
+
+    def run():
+        if loss == "readout":
+            O, lse = swvr.softmax_readout(*xs, chunk_size=256)
+            return O.sin().sum() + lse.cos().sum()
+        w = weight if loss == "weighted" else None
+        return swvr.softmax_readout_mse(*xs[:3], target, xs[3], weight=w, chunk_size=256)
+    wrt = [xs[0], xs[2], xs[3]]
+    want, out = torch.autograd.grad(run(), wrt), run()
+    with SeenOps() as seen:
+        got = torch.autograd.grad(out, wrt)
+    assert "swvr.chunked_bwd.default" in seen.names and "swvr.chunked_fwd.default" not in seen.names
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_saved_tensor_hooks_and_a_second_derivative():
     xs = make(20, 64, 300, 16, torch.float32)
     target = torch.randn(20, 16, device="cuda")
