@@ -1010,10 +1010,13 @@ constexpr int64_t kFewTokens = 768;
 // non-finite values first.  Past it the few-token kernel runs over the active tokens' positions.
 constexpr int64_t kFewTokensActive = 512, kFewTokensActiveF32 = 128;
 
+// Whether a call is planned for the few-token forward.
+bool takes_few(int dtype, int64_t N) { return dtype != kFP8 && (dtype == kF32 || N <= kFewTokens); }
+
 // Tile, split and workspace (from offset off on) of the few-token forward for one pass of Dw columns:
 // vocabulary runs of whole 32-row groups.
 void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, size_t off, FwdPlan* plan) {
-  plan->few = dtype != kFP8 && (dtype == kF32 || N <= kFewTokens);
+  plan->few = takes_few(dtype, N);
   if (!plan->few) return;
   const bool two = dtype != kF32;
   plan->few_DP = !two && Dw <= 32 ? 32 : Dw <= 64 ? 64 : Dw <= 128 ? 128 : 256;
@@ -1170,13 +1173,14 @@ bool fwd_plan(int dtype, int64_t N, int64_t K, int64_t V, int64_t D, FwdPlan* pl
   // least two vocabulary tiles per split.
   int n_split = 1;
   if (plan->n_tb > 0) {
-    const int target = 1024;
+    // (a call planned for the few-token forward comes here for rows too far apart for it alone: one round)
+    const int target = takes_few(dtype, N) ? kFwdRound : 1024;
     n_split = (target + plan->n_tb - 1) / plan->n_tb;
     const int max_split = plan->n_vt / 2 > 1 ? plan->n_vt / 2 : 1;
     if (n_split > max_split) n_split = max_split;
     if (n_split < 1) n_split = 1;
     // (the e4m3 forward's P is relative to the running maximum, so it keeps at least the rule's splits)
-    if (!active && tbytes == 2)
+    if (!active && tbytes == 2 && !takes_few(dtype, N))
       n_split = balanced_split(plan->n_tb, plan->n_vt, n_split, dtype == kFP8 ? n_split : 1,
                                fwd_cost(K, DP, BM, WV));
   }
@@ -1306,32 +1310,12 @@ __global__ __launch_bounds__(256) void fwd_w_scan_kernel(const Src* __restrict__
 }
 
 // The few-token forward's token blocks and vocabulary runs (few_runs) for the count, into n_act[3],
-// n_act[4]; one wave, a candidate per lane.
+// n_act[4].
 __global__ __launch_bounds__(64) void fwd_few_grid_kernel(int* __restrict__ n_act, int BM, int grp) {
-  const int n = n_act[0], tb = (n + BM - 1) / BM;
-  int64_t best = INT64_MAX;
-  int pick = 1;
-  if (tb > 0)
-    for (int s = 1 + (int)threadIdx.x; s <= few_runs_max(tb, grp); s += 64) {
-      const int64_t t = few_span(tb, grp, s);
-      if (t < best) {
-        best = t;
-        pick = s;
-      }
-    }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const int64_t t = __shfl_xor(best, o);
-    const int q = __shfl_xor(pick, o);
-    if (t < best || (t == best && q < pick)) {
-      best = t;
-      pick = q;
-    }
-  }
-  if (threadIdx.x == 0) {
-    n_act[3] = tb;
-    n_act[4] = pick;
-  }
+  if (threadIdx.x != 0) return;
+  const int tb = (n_act[0] + BM - 1) / BM;
+  n_act[3] = tb;
+  n_act[4] = few_runs(tb, grp);
 }
 
 // Everything of the active-token forward before its passes: the parameter flags (bad[0..1], set

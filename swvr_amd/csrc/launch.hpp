@@ -157,10 +157,19 @@ __host__ __device__ inline int few_runs_max(int64_t n_tb, int64_t grp) {
   const int64_t m = kFewRounds * kFwdRound / (n_tb > 0 ? n_tb : 1), c = m < grp ? m : grp;
   return c < 1 ? 1 : (int)c;
 }
-inline int few_runs(int64_t n_tb, int64_t grp) {
+// Within a number of rounds the span falls with the length of the longest run alone, so the candidates are
+// the most runs that each number of rounds holds, brought down to the fewest with the same longest run (all
+// counts tried one by one took the host 5 us of a one-token call, twice).
+__host__ __device__ inline int few_runs(int64_t n_tb, int64_t grp) {
+  const int64_t most = few_runs_max(n_tb, grp);
   int best = 1;
-  for (int s = 2; s <= few_runs_max(n_tb, grp); ++s)
-    if (few_span(n_tb, grp, s) < few_span(n_tb, grp, best)) best = s;
+  for (int64_t r = 1; r <= kFewRounds; ++r) {
+    const int64_t fit = r * kFwdRound / (n_tb > 0 ? n_tb : 1), s = fit < most ? fit : most;
+    if (s < 1 || grp < 1) continue;
+    const int64_t run = (grp + s - 1) / s;
+    const int64_t fewest = (grp + run - 1) / run;
+    if (few_span(n_tb, grp, fewest) < few_span(n_tb, grp, best)) best = (int)fewest;
+  }
   return best;
 }
 hipError_t fwd_few_launch(int dtype, const FwdFewParams& p, hipStream_t stream);

@@ -59,3 +59,32 @@ def test_inline_assembly_declares_the_scalar_condition_code():
                 checked += 1
                 assert '"scc"' in body, f"{name}: inline assembly writes SCC without declaring it: {code[:80]}"
     assert checked >= 2
+
+
+RUNS_MAIN = r"""
+#include "launch.hpp"
+#include <stdio.h>
+using namespace swvr;
+int main() {
+  long n = 0;
+  for (int64_t tb = 0; tb <= 1100; tb = tb < 40 ? tb + 1 : tb + 1 + tb / 9)
+    for (int64_t grp = 0; grp < 9000; grp = grp < 100 ? grp + 1 : grp + 1 + grp / 23, ++n) {
+      int best = 1;
+      for (int s = 2; s <= few_runs_max(tb, grp); ++s)
+        if (few_span(tb, grp, s) < few_span(tb, grp, best)) best = s;
+      if (few_runs(tb, grp) != best) return printf("%d blocks, %d groups: %d, not %d\n", (int)tb, (int)grp,
+                                                   few_runs(tb, grp), best), 1;
+    }
+  return n < 5000;
+}
+"""
+
+
+def test_vocabulary_runs_are_the_best_of_all_counts(tmp_path):
+    """The few-token forward's split (few_runs), from a few candidates, against every count tried."""
+    import subprocess
+    (tmp_path / "runs.cpp").write_text(RUNS_MAIN)
+    exe = str(tmp_path / "runs")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{build.CSRC}",
+                    str(tmp_path / "runs.cpp"), "-o", exe], check=True)
+    assert subprocess.run([exe]).returncode == 0
