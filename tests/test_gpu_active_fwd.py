@@ -207,6 +207,25 @@ def test_non_finite_inputs_give_the_reference_nans(kind, reduction):
     same_nan_pattern_and_values(got, want)
 
 
+# the same rules on the other routes: one pass over every token (few 2-byte tokens), the few-token kernel over
+# positions with W scanned for non-finite values (fp32, 2-byte to 768), and the general kernels with W flagged
+# while it is packed (2-byte past that, and an fp32 W under autocast)
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("dtype,N,amp", [(torch.bfloat16, 64, False), (torch.float32, 200, False),
+                                         (torch.bfloat16, 600, False), (torch.float32, 600, True),
+                                         (torch.float16, 1000, False), (torch.float32, 1000, True)])
+def test_non_finite_inputs_give_the_reference_nans_on_every_route(kind, dtype, N, amp):
+    K, V, D = 40, 301, 8
+    h, W, E, b = inputs(N, K, V, D, dtype, seed=11)
+    target = torch.randn(N, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(12))
+    w = mask(N, 0.3, seed=13)
+    h, W, E, b, target, w, scale = poison(kind, h, W, E, b, target, w)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+        got = swvr.softmax_readout_mse(h, W, E, target, b, weight=w, z_loss_weight=1e-3, reduction="none",
+                                       logit_scale=scale)
+    same_nan_pattern_and_values(got, composite(h, W, E, b, target, w, 1e-3, "none", scale))
+
+
 def test_the_loss_takes_the_active_forward_only_where_it_is_exact():
     from swvr_amd.api import _skips_zero_weight
     h, W, E, b = inputs(64, 32, 300, 8, torch.bfloat16)

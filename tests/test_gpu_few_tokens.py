@@ -123,8 +123,10 @@ def test_few_token_forward(dtype, N, K, V, D):
     hd, Wd, Ed = (x.to(cd).double() for x in (h, W, E))
     S = 0.7 * (hd @ Wd.T) + b.double()
     want_O, want_lse = torch.softmax(S, -1) @ Ed, torch.logsumexp(S, -1)
-    bar = 1e-5 if cd == torch.float32 else 1e-2
-    assert rel_err(O, want_O) <= bar and rel_err(lse, want_lse) <= bar, (rel_err(O, want_O), rel_err(lse, want_lse))
+    # P alone is rounded beside the operands: the rms of a rounding to 8 or 11 bits is 1.6e-3 or 2e-4, which
+    # averages out over the rows but for the few that dominate; lse is a 32-bit sum
+    bar = {torch.float32: 1e-5, torch.bfloat16: 2e-3, torch.float16: 2.5e-4}[cd]
+    assert rel_err(O, want_O) <= bar and rel_err(lse, want_lse) <= 1e-5, (rel_err(O, want_O), rel_err(lse, want_lse))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -181,7 +183,8 @@ def test_weighted_few_token_forward_zeroes_the_rows_of_zero_weight(dtype, N):
 
 
 # embeddings wider than one pass whose last pass runs on a narrower kernel (64, 128 columns, whole
-# passes beside), with token counts whose vocabulary splits are balanced and ones where they are not
+# passes beside), with token counts whose vocabulary splits are balanced and ones where they are not; in
+# fp32 the passes are the few-token kernel's (the general kernels': the test of far-apart rows below)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("N,K,V,D", [(2500, 64, 9000, 300), (1100, 96, 3000, 257), (3000, 40, 4097, 640),
                                      (1030, 64, 300, 384)])
@@ -193,6 +196,31 @@ def test_last_pass_of_wide_embeddings_on_a_narrower_kernel(dtype, N, K, V, D):
     for sl in (slice(0, D // 256 * 256), slice(D // 256 * 256, D)):
         assert sl.start == sl.stop or rel_err(O[:, sl], torch.softmax(S, -1) @ E.double()[:, sl]) <= bar
     assert rel_err(lse, torch.logsumexp(S, -1)) <= bar
+
+
+# rows of W or E further apart than the few-token kernel's 32-bit offsets reach (16 MB and more): packed for
+# the general kernels, which fp32 and few tokens take for nothing else
+@pytest.mark.parametrize("dtype,amp,N,D,far", [
+    (torch.bfloat16, False, 20, 24, "W"), (torch.bfloat16, False, 200, 64, "E"), (torch.float16, False, 40, 300, "W"),
+    (torch.float32, True, 33, 64, "W"), (torch.float32, False, 20, 24, "W"), (torch.float32, False, 300, 140, "W"),
+    (torch.float32, False, 130, 64, "E")])
+def test_rows_far_apart_take_the_general_kernels(dtype, amp, N, D, far):
+    from swvr_amd import _ops
+    K, V = 72, 130
+    h, W, E, b = make(N, K, V, D, dtype, requires_grad=False)
+    step = 2**24 // W.element_size() + 8   # 128 such rows: 2^31 bytes, the line
+    x = W if far == "W" else E
+    x2 = torch.empty((V - 1) * step + x.shape[1], dtype=dtype, device="cuda").as_strided(x.shape, (step, 1)).copy_(x)
+    Wf, Ef = (x2, E) if far == "W" else (W, x2)
+    weight = (torch.arange(N, device="cuda") % 3 > 0).float()
+
+    def call(W, E):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            cdt = torch.bfloat16 if amp else dtype
+            return (*swvr.softmax_readout(h, W, E, b), *_ops._forward_active(h, W, E, b, weight, 1.0, 8192, cdt))
+    bar = 1e-5 if dtype == torch.float32 and not amp else 2e-3
+    for a, r in zip(call(Wf, Ef), call(W, E)):
+        assert rel_err(a, r) <= bar
 
 
 # the few-token kernel over the active tokens' positions (fp32 at any size, 2-byte types between 512 and

@@ -42,8 +42,8 @@ def test_sums_over_a_long_vocabulary(dtype, N, D):
     e_l = rel_err(l[rows].double() * torch.exp(m[rows].double() - want_lse), torch.ones_like(want_lse))
     e_lse, e_O = rel_err(lse[rows], want_lse), rel_err(O[rows], want_O)
     print(f"\n{dtype} {N}: l {e_l:.2e} lse {e_lse:.2e} O {e_O:.2e}")
-    assert e_l <= 2 ** -23 and e_lse <= 2 ** -23 and e_O <= {torch.float32: 4e-6, torch.bfloat16: 1.2e-3,
-                                                         torch.float16: 1.5e-4}[dtype]
+    assert e_l <= 2 ** -23 and e_lse <= 2 ** -23 and e_O <= {torch.float32: 4e-6, torch.bfloat16: 1e-3,
+                                                         torch.float16: 1.2e-4}[dtype]
 
 
 # E near the largest finite values under scores that fall by 20 after the first row and, in the middle, rise
