@@ -1048,6 +1048,8 @@ void few_plan(int dtype, int64_t N, int64_t V, int64_t Dw, bool active, size_t o
 }
 
 // Whether the call takes the few-token forward: planned so, and 32-bit offsets reach 128 rows of W and E.
+// Rows 16 MB and more apart go to the general kernels, whatever the type and the number of tokens; the
+// workspace, sized before the strides are known, holds either route.
 bool few_fits(const FwdPlan& plan, const FwdParams& p, int dtype) {
   const int64_t esz = dtype == kF32 ? 4 : 2, wsz = p.w_f32 ? 4 : esz, lim = (int64_t)1 << 31;
   return plan.few && p.ldw * wsz * 128 < lim && p.lde * esz * 128 < lim;

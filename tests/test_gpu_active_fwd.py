@@ -91,7 +91,7 @@ def test_active_forward_matches_the_oracle(cdt, N, K, V, D, frac):
 
 def test_halving_the_active_blocks_resplits_the_vocabulary():
     """20000 tokens in 79 blocks, half of them masked: about 40 active blocks, so
-    active_grid doubles the vocabulary splits; the partials then span the same buffer."""
+    the split picked on the device grows; the partials then span the same buffer."""
     N, K, V, D = 20000, 128, 4096, 64
     h, W, E, b = inputs(N, K, V, D, torch.bfloat16, seed=5)
     for frac in (0.5, 0.75, 0.02):
