@@ -109,6 +109,20 @@ def test_a_backward_run_under_a_mode_shows_its_op(loss):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+def test_calls_without_a_chunk_agree_compiled_and_eager():
+    """Eager calls of few tokens stage more rows at a time than the ops' 8192, compiled ones those: the same
+    gradients but for the order of gh's sums."""
+    xs = make(40, 64, 20000, 16, torch.float32)
+    target = torch.randn(40, 16, device="cuda")
+    fn = lambda h: swvr.softmax_readout_mse(h, *xs[1:3], target, xs[3])
+    torch._dynamo.reset()
+    loss_c, loss_e = torch.compile(fn, fullgraph=True)(xs[0]), fn(xs[0])
+    assert _ops._rows_staged(None, 2, 2, 40, 64, 20000, 16, True) > 8192
+    assert torch.equal(loss_c, loss_e)
+    for a, b in zip(torch.autograd.grad(loss_c, xs), torch.autograd.grad(loss_e, xs)):
+        assert (a - b).norm() <= 1e-5 * b.norm()
+
+
 def test_saved_tensor_hooks_and_a_second_derivative():
     xs = make(20, 64, 300, 16, torch.float32)
     target = torch.randn(20, 16, device="cuda")
